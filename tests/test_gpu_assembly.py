@@ -162,3 +162,18 @@ def test_several_elements_per_workgroup(gpu, p, nel):
     assert np.abs(K[idx].cpu().numpy() - Ko).max() <= 1e-12 * scale
     assert np.abs(Kv[idx].cpu().numpy() - Ko).max() <= 1e-12 * scale
     asm.close()
+
+
+@pytest.mark.parametrize("p,ng", [(1, 2), (1, 9), (3, 5), (4, 5)])
+def test_load_point_chunks_match_oracle(gpu, p, ng):
+    """Every load type with 4 to 729 points per load and 8 to 125 nodes: each split of a load's
+    points over the lanes (16, 8 and 4 lanes per point), points past one 64-point chunk and node
+    counts on both sides of the splits of the node sums (F within 1e-12 of its maximum: sums of
+    at most 729 products of O(1) factors in 64 bits)."""
+    print("[case] loads p=%d ng=%d" % (p, ng), flush=True)
+    bp = make_box_patch(nel=(2, 2, 1), p=p, seed=6, ngauss=ng)
+    a = all_face_loads(bp)
+    from yeti_amd.stiffmtrx_elemstorage import sys_linmat_lindef_static
+    F = sys_linmat_lindef_static(**a)[3]
+    F0 = O.oracle_sys_linmat((), kwargs=a)[3]
+    assert np.abs(F - F0).max() <= 1e-12 * np.abs(F0).max()
