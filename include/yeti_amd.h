@@ -174,8 +174,7 @@ int32_t yeti_asm_volume_grad(yeti_asm *h, double *vol, double *g, void *stream);
  * with the external term restricted to what the reference computes: the centrifugal body loads
  * (type 101), whose axis points the k-th such load reads at values 6k+1..6k+6 of
  * load_additionalInfos as the reference does; its surface-load term is a stub (zero) there and
- * here. activeDir plays no part (the reference's solid routine does not read it). Synchronises
- * `stream` once (the polarisation scales). */
+ * here. activeDir plays no part (the reference's solid routine does not read it). */
 int32_t yeti_grad_lin_elast_work(yeti_asm *h, const double *SOL, const double *ADJ, int32_t nadj, int32_t computeWint,
                                  int32_t computeWext, double *gradWint, double *gradWext, void *stream);
 /* Right-hand side only (concentrated, surface and body loads). */

@@ -136,3 +136,30 @@ def test_gpu_gradvibration_an_dropin():
     go = O.oracle_grad_vibration(d, V, w)
     assert g.shape == (2, 3, int(d["nb_cp"])) and g.flags.f_contiguous
     assert np.abs(g - go).max() <= 1e-11 * np.abs(go).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("nel,p", [((47, 47, 45), 1), ((5, 3, 1), 2), ((24, 23, 23), 3), ((3, 1, 1), 4)])
+def test_gpu_gradient_waves_and_strides(nel, p):
+    """The factorised kernel where a wave carries several elements (p = 1, 2) with a last wave that
+    is partly past the end, and where the elements outnumber the launched waves (p = 1, 3: more
+    than 3072 workgroups' worth), so that a wave walks several: against the oracle (1e-11 of the
+    maximum), and the state-adjoint form with the adjoint equal to the state against the
+    strain-energy form (1e-12: the same sums, rounded differently)."""
+    import torch
+    from yeti_amd.assembly import Assembler
+    print("[case] gradient waves %s p=%d" % (nel, p), flush=True)
+    d = dict(make_box_patch(nel=nel, p=p, seed=9, rho=7.8e-9).args)
+    ncp = int(d["nb_cp"])
+    V = np.random.default_rng(3).standard_normal((1, 3, ncp))
+    asm = Assembler(d)
+    try:
+        g = asm.run_vib_grad(V, [2e6]).cpu().numpy()
+        u = torch.from_numpy(np.ascontiguousarray(V[0].T.reshape(-1))).cuda()
+        e = asm.strain_energy_grad(u)
+        w, _ = asm.grad_lin_elast_work(u, u.reshape(1, -1), True, False)
+        assert float((w[0] - e).abs().max()) <= 1e-12 * float(e.abs().max())
+    finally:
+        asm.close()
+    go = O.oracle_grad_vibration(d, V, np.array([2e6]))
+    assert np.abs(g - go).max() <= 1e-11 * np.abs(go).max()

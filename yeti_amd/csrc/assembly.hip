@@ -95,8 +95,8 @@ void gauss_rule_host(int n, double *x, double *w) { gauss_legendre(n, x, w); }
 // Device: non-zero B-splines of degree P and first derivatives at u for 0-based span i
 // (Cox-de Boor triangle + closed-form derivative; the contract of dersbasisfuns.f90:30-131).
 template <int P>
-__device__ inline void bspline_ders(int i, double u, const double *__restrict__ U, double *N,
-                                    double *dN) {
+__host__ __device__ inline void bspline_ders(int i, double u, const double *__restrict__ U, double *N,
+                                             double *dN) {
     double left[P + 1], right[P + 1], cur[P + 1], low[P + 1];
     cur[0] = 1.0;
     low[0] = 1.0;
@@ -135,6 +135,7 @@ __device__ inline void bspline_ders(int i, double u, const double *__restrict__ 
 }
 
 #include "elem_kernel.hpp"
+#include "shape_grad.hpp"
 
 // ------------------------------------------------------------------------------------------
 // Right-hand side of loaded elements (UELMAT.f90:121-223): body loads 101/102 at the volume
@@ -731,6 +732,9 @@ struct PatchDev {
     double lam, mu, rho;
     bool u1;
     DevBuf<double> U[3];
+    // 1D basis tables per knot span, padded to tab_n = max degree + 1 functions (shape_grad.hpp);
+    DevBuf<double> tab[3];
+    int tab_n = 0;
     DevBuf<int32_t> ien, nijk, elems;
     DevBuf<double> weight;
     DevBuf<int64_t> offs;
@@ -766,17 +770,17 @@ struct yeti_asm {
     std::vector<hipEvent_t> ev;
     int32_t ev_used = 0;
     int32_t n_loaded_total = 0;
-    // natural-frequency gradient (built on first use): CP -> element-node entries of the active
-    // U1 elements in CSR form, per-entry and per-element partials, the per-mode mass
+    // shape gradients (built on first use): CP -> element-node entries of the active U1 elements
+    // in CSR form, the per-entry partials, the masses per workgroup and per pair
     yeti::DevBuf<int32_t> vib_ptr;
-    yeti::DevBuf<int64_t> vib_ent;
+    yeti::DevBuf<int32_t> vib_ent;
     yeti::DevBuf<double> vib_eg, vib_em, vib_mass;
-    yeti::DevBuf<double> vol_u;    // translation field of the volume gradient
     // gradLinElastWork_AN: offsets of the centrifugal loads' axis points in load_additionalInfos
     // as the reference reads them (the k-th load of type 101 at 6k), and the work buffers
     yeti::DevBuf<int32_t> add_off_ref;
     bool ref_infos_ok = true;
-    yeti::DevBuf<double> gw_fields, gw_grads, gw_vec, gw_vec2, gw_sums;
+    bool any_centrifugal = false;   // a load of type 101
+    yeti::DevBuf<double> gw_vec, gw_vec2;
     int64_t vib_nent = -1, vib_nslot = 0;
     ~yeti_asm() {
         for (auto *p : patches) delete p;
@@ -823,6 +827,38 @@ static bool kernel_available(int p0, int p1, int p2, int ng) {
     if (mfma_kernel_available(p0, p1, p2, ng)) return true;
     return p0 >= 1 && p1 >= 1 && p2 >= 1 && p0 <= 4 && p1 <= 4 && p2 <= 4 && (p0 + 1) * (p1 + 1) * (p2 + 1) <= 64 &&
            ng >= 1 && ng <= MAX_NG;
+}
+
+// Table of one direction for the factorised gradient kernel: n = degree + 1 functions of each
+// knot span with elements, padded to N, at N Gauss points (layout: shape_grad.hpp)
+template <int P>
+static void basis_table_p(const double *U, int nkv, int N, std::vector<double> &tab) {
+    const int rec = 2 * N * N + 2;
+    double gx[MAX_NG], gw[MAX_NG], B[P + 1], dB[P + 1];
+    gauss_legendre(N, gx, gw);
+    tab.assign((size_t)rec * std::max(nkv - 1, 1), 0.0);
+    for (int i = P; i + P + 1 < nkv; ++i) {
+        const double u0 = U[i], u1 = U[i + 1];
+        if (!(u1 > u0)) continue;
+        double *t = tab.data() + (size_t)rec * i;
+        for (int g = 0; g < N; ++g) {
+            bspline_ders<P>(i, ((u1 - u0) * gx[g] + (u1 + u0)) * 0.5, U, B, dB);
+            for (int r = 0; r <= P; ++r) {   // reversed local index (shap.f90:94-119)
+                t[g * N + P - r] = B[r];
+                t[N * N + g * N + P - r] = dB[r];
+            }
+        }
+        t[2 * N * N] = 0.5 * (u1 - u0);
+    }
+}
+
+static void basis_table(int p, const double *U, int nkv, int N, std::vector<double> &tab) {
+    switch (p) {
+    case 1: basis_table_p<1>(U, nkv, N, tab); break;
+    case 2: basis_table_p<2>(U, nkv, N, tab); break;
+    case 3: basis_table_p<3>(U, nkv, N, tab); break;
+    default: basis_table_p<4>(U, nkv, N, tab); break;
+    }
 }
 
 static int device_cu_count() {
@@ -1521,55 +1557,32 @@ __device__ inline void bspline_ders_rt(int i, int p, double u, const double *__r
     }
 }
 
-// ---------------------------------------------------------------------------------------
-// Natural-frequency shape gradient (gradvibration_fullAN.f:22-189 with gradUELMASSMAT1,
-// gradUELMASSMAT_solid.f:22-332), solid patches, up to VIB_MAXF modes per launch. For mode f with
-// eigenvalue lambda_f and eigenvector u, element e adds to its node a
-//   g_a[m] = sum_q dv_q [ (eps:sig - lambda_f rho |u|^2) dR_a/dx_m - 2 sum_ik sig_ik du_i/dx_m dR_a/dx_k ],
-// the derivative of u^T (K - lambda_f M) u with respect to control point a (the reference writes
-// the same derivative in the covariant basis as its Jacobian, strain and metric terms), and the
-// mass rho |u|^2 dv; the CP gradient is the sum over elements divided by the total mass per mode.
-// One 256-thread workgroup per active element, Gauss points in chunks of VQC:
+// Shape gradients of models with other than max(p) + 1 Gauss points per direction: run-time
+// degrees and order, one 256-thread workgroup per active element, Gauss points in chunks of VQC:
 //   1. bases, one thread per (point, direction);
 //   2. W, dW and dx/du of a point by 256 / VQC threads and a shuffle sum, then du/dx and dv;
 //   3. R and dR/dx of every (node, point) of the chunk in LDS;
-//   4. per (point, mode): u, du/dx, sig, the tensor dv (W' I - 2 (du/dx)^T sig) and the mass;
-//   5. per (node, mode): g += tensor . dR/dx, accumulated over the chunks in the registers of the
-//      (node, mode) pair's thread.
-constexpr int VIB_MAXF = 4, VQC = 16;
+//   4. per (point, pair): the tensor T[m][k] and the mass;
+//   5. per (node, pair): g += tensor . dR/dx, accumulated over the chunks in the registers of the
+//      (node, pair)'s thread.
+constexpr int VQC = 16;
 
-struct VibModes {
-    const double *vect;            // (nb_frq, 3, nb_cp) column-major
-    int32_t nf_total, f0, nf;      // modes f0 .. f0 + nf - 1 of nf_total
-    double vals[VIB_MAXF];
-    double scale;                  // the CP sums are multiplied by scale ...
-    int32_t normalize;             // ... and divided by each mode's mass when set
-    int32_t unit_density;          // density 1 in place of the patches' (volume)
-};
-
-// RT = false: degree P in every direction and NG points (compile-time); RT = true: the degrees and
-// Gauss order of `dg` at run time, P and GEN_MAXN bounding the arrays.
-struct VibDegrees {
+struct GradDegrees {
     int p[3];
     int ng;
 };
 
-// waves per SIMD the kernel is compiled for: at p = 3 three (its LDS allows three workgroups per
-// CU once the node sums are in registers), at p = 2 four, elsewhere what the registers give
-template <int P, bool RT>
-constexpr int vib_wpe() { return RT ? 1 : P == 3 ? 3 : P == 2 ? 4 : 1; }
-
-template <int P, int NG, bool RT = false>
-__global__ void __launch_bounds__(256) __attribute__((amdgpu_waves_per_eu(vib_wpe<P, RT>())))
-vib_grad_kernel(PatchArgs pa, double rho, VibModes vm, int64_t ebase,
-                                                       int64_t mbase, double *__restrict__ eg,
-                                                       double *__restrict__ em, VibDegrees dg = VibDegrees{}) {
-    constexpr int NP1 = P + 1, NN = RT ? GEN_MAXN : NP1 * NP1 * NP1, G = 256 / VQC;
-    const int p0 = RT ? dg.p[0] : P, p1 = RT ? dg.p[1] : P, p2 = RT ? dg.p[2] : P;
-    const int n0 = p0 + 1, n1 = p1 + 1, nn = RT ? n0 * n1 * (p2 + 1) : NN;
-    const int ng = RT ? dg.ng : NG, NQ = ng * ng * ng;
+template <int KIND>
+__global__ void __launch_bounds__(256) shape_grad_rt_kernel(PatchArgs pa, GradFields gf, GradDegrees dg,
+                                                            int64_t ebase, double *__restrict__ eg,
+                                                            double *__restrict__ em) {
+    constexpr int P = GEN_MAXP, NP1 = P + 1, NN = GEN_MAXN, G = 256 / VQC;
+    const int p0 = dg.p[0], p1 = dg.p[1], p2 = dg.p[2];
+    const int n0 = p0 + 1, n1 = p1 + 1, nn = n0 * n1 * (p2 + 1);
+    const int ng = dg.ng, NQ = ng * ng * ng;
+    constexpr int NFLD = KIND == GRAD_VOLUME ? 1 : KIND == GRAD_PAIRS ? VIB_MAXF + 1 : VIB_MAXF;
     __shared__ double xw[NN][4];
-    __shared__ double uf[VIB_MAXF][NN][3];
+    __shared__ double uf[NFLD][NN][3];
     __shared__ double Bq[VQC][3][NP1], dBq[VQC][3][NP1];
     __shared__ double gq[VQC][14];     // du/dx (9, [c][k] = du_c/dx_k), dv, 1/W, dW/du / W (3)
     __shared__ double Rx[NN][VQC][4];  // R, dR/dx
@@ -1577,7 +1590,7 @@ vib_grad_kernel(PatchArgs pa, double rho, VibModes vm, int64_t ebase,
     __shared__ double mpart[VQC][VIB_MAXF];
     __shared__ double hel[3];
     const int t = threadIdx.x;
-    const int nf = vm.nf;
+    const int nf = KIND == GRAD_VOLUME ? 1 : gf.nf;
     const int qq = t / G, part = t % G;
     for (int64_t gi = blockIdx.x; gi < pa.n_active; gi += gridDim.x) {
         const int e = pa.elems[gi];
@@ -1588,16 +1601,18 @@ vib_grad_kernel(PatchArgs pa, double rho, VibModes vm, int64_t ebase,
             xw[a][1] = pa.coords[3 * cp + 1];
             xw[a][2] = pa.coords[3 * cp + 2];
             xw[a][3] = pa.weight[(int64_t)nn * e + a];
-            for (int f = 0; f < nf; ++f)
-                for (int c = 0; c < 3; ++c)
-                    uf[f][a][c] = vm.vect[(vm.f0 + f) + (int64_t)vm.nf_total * (c + 3 * cp)];
+            if (KIND != GRAD_VOLUME)
+                for (int c = 0; c < 3; ++c) {
+                    for (int f = 0; f < nf; ++f) uf[f][a][c] = gf.fk[(gf.k0 + f) + (int64_t)gf.nk * (c + 3 * cp)];
+                    if (KIND == GRAD_PAIRS) uf[NFLD - 1][a][c] = gf.f0[c + 3 * cp];
+                }
         }
-        // this thread's node sums: (node, mode) x = t + 256 s, a = x mod nn, f = x / nn
+        // this thread's node sums: (node, pair) x = t + 256 s, a = x mod nn, f = x / nn
         constexpr int GSL = (NN * VIB_MAXF + 255) / 256;
         double gr[GSL][3];
 #pragma unroll
         for (int s = 0; s < GSL; ++s) gr[s][0] = gr[s][1] = gr[s][2] = 0.0;
-        double macc = 0.0;   // this thread's (point, mode) share of the element mass
+        double macc = 0.0;   // this thread's (point, pair) share of the element mass
         for (int q0 = 0; q0 < NQ; q0 += VQC) {
             const int nq = NQ - q0 < VQC ? NQ - q0 : VQC;
             __syncthreads();
@@ -1610,20 +1625,11 @@ vib_grad_kernel(PatchArgs pa, double rho, VibModes vm, int64_t ebase,
                 const double u0 = U[span1 - 1], u1 = U[span1];
                 const double u = ((u1 - u0) * pa.g.x[gd] + (u1 + u0)) * 0.5;
                 double N[NP1], dN[NP1];
-                if constexpr (RT) {
-                    const int pd = d == 0 ? p0 : d == 1 ? p1 : p2;
-                    bspline_ders_rt<P>(span1 - 1, pd, u, U, N, dN);
-                    for (int i = 0; i <= pd; ++i) {
-                        Bq[qq][d][i] = N[pd - i];
-                        dBq[qq][d][i] = dN[pd - i];
-                    }
-                } else {
-                    bspline_ders<P>(span1 - 1, u, U, N, dN);
-#pragma unroll
-                    for (int i = 0; i < NP1; ++i) {
-                        Bq[qq][d][i] = N[P - i];
-                        dBq[qq][d][i] = dN[P - i];
-                    }
+                const int pd = d == 0 ? p0 : d == 1 ? p1 : p2;
+                bspline_ders_rt<P>(span1 - 1, pd, u, U, N, dN);
+                for (int i = 0; i <= pd; ++i) {
+                    Bq[qq][d][i] = N[pd - i];
+                    dBq[qq][d][i] = dN[pd - i];
                 }
                 if (qq == 0) hel[d] = 0.5 * (u1 - u0);
             }
@@ -1711,13 +1717,13 @@ vib_grad_kernel(PatchArgs pa, double rho, VibModes vm, int64_t ebase,
                 for (int kk = 0; kk < 4; ++kk) Rx[a][c][kk] = r4[kk];
             }
             __syncthreads();
-            // 4. per (point, mode): u, du/dx, stress, the tensor and the mass; the nodes of a
-            // (point, mode) pair are split over 4 adjacent lanes and their sums added by shuffles
+            // 4. per (point, pair): the fields, stresses, the tensor and the mass; the nodes of a
+            // (point, pair) are split over 4 adjacent lanes and their sums added by shuffles
             {
                 const int pr = t >> 2, part4 = t & 3, c = pr % VQC, f = pr / VQC;
                 const bool act = f < nf && c < nq;
-                double u[3] = {0.0, 0.0, 0.0}, D[3][3] = {};   // D[i][k] = du_i/dx_k
-                if (act) {
+                double u[3] = {0.0, 0.0, 0.0}, D[3][3] = {}, H[3][3] = {};   // D[i][k] = dv_i/dx_k, H: field 0
+                if (KIND != GRAD_VOLUME && act) {
 #pragma unroll 1
                     for (int a = part4; a < nn; a += 4) {
                         const double R = Rx[a][c][0], g0 = Rx[a][c][1], g1 = Rx[a][c][2], g2 = Rx[a][c][3];
@@ -1728,6 +1734,12 @@ vib_grad_kernel(PatchArgs pa, double rho, VibModes vm, int64_t ebase,
                             D[i][0] += ua * g0;
                             D[i][1] += ua * g1;
                             D[i][2] += ua * g2;
+                            if (KIND == GRAD_PAIRS) {
+                                const double u0 = uf[NFLD - 1][a][i];
+                                H[i][0] += u0 * g0;
+                                H[i][1] += u0 * g1;
+                                H[i][2] += u0 * g2;
+                            }
                         }
                     }
                 }
@@ -1737,40 +1749,50 @@ vib_grad_kernel(PatchArgs pa, double rho, VibModes vm, int64_t ebase,
                     for (int i = 0; i < 3; ++i) {
                         u[i] += __shfl_xor(u[i], o, 64);
 #pragma unroll
-                        for (int k = 0; k < 3; ++k) D[i][k] += __shfl_xor(D[i][k], o, 64);
+                        for (int k = 0; k < 3; ++k) {
+                            D[i][k] += __shfl_xor(D[i][k], o, 64);
+                            if (KIND == GRAD_PAIRS) H[i][k] += __shfl_xor(H[i][k], o, 64);
+                        }
                     }
                 }
+                if (KIND == GRAD_MODES)
+#pragma unroll
+                    for (int i = 0; i < 3; ++i)
+#pragma unroll
+                        for (int k = 0; k < 3; ++k) H[i][k] = D[i][k];
                 if (part4 == 0 && f < nf) {
                     double T[9] = {0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 0.0};
                     if (c < nq) {
                         const double lam = pa.lam, mu = pa.mu, dv = gq[c][9];
-                        const double tr = D[0][0] + D[1][1] + D[2][2];
-                        double sig[3][3], W = 0.0;
+                        const double td = lam * (D[0][0] + D[1][1] + D[2][2]), th = lam * (H[0][0] + H[1][1] + H[2][2]);
+                        double sd[3][3], sh[3][3], W = 0.0;
 #pragma unroll
                         for (int i = 0; i < 3; ++i)
 #pragma unroll
                             for (int k = 0; k < 3; ++k) {
-                                const double eik = 0.5 * (D[i][k] + D[k][i]);
-                                sig[i][k] = 2.0 * mu * eik + (i == k ? lam * tr : 0.0);
-                                W += eik * sig[i][k];
+                                sd[i][k] = mu * (D[i][k] + D[k][i]) + (i == k ? td : 0.0);
+                                sh[i][k] = mu * (H[i][k] + H[k][i]) + (i == k ? th : 0.0);
+                                W += sh[i][k] * D[i][k];
                             }
-                        const double uu = u[0] * u[0] + u[1] * u[1] + u[2] * u[2];
-                        const double Wp = W - vm.vals[f] * rho * uu;
+                        const double uu = KIND == GRAD_MODES ? gf.rho * (u[0] * u[0] + u[1] * u[1] + u[2] * u[2])
+                                                             : KIND == GRAD_VOLUME ? 1.0 : 0.0;
+                        const double Wp = KIND == GRAD_VOLUME ? 1.0 : KIND == GRAD_MODES ? W - gf.vals[f] * uu : W;
 #pragma unroll
                         for (int m = 0; m < 3; ++m)
 #pragma unroll
                             for (int k = 0; k < 3; ++k) {
                                 double v = m == k ? Wp : 0.0;
-                                v -= 2.0 * (D[0][m] * sig[0][k] + D[1][m] * sig[1][k] + D[2][m] * sig[2][k]);
+#pragma unroll
+                                for (int i = 0; i < 3; ++i) v -= D[i][m] * sh[i][k] + H[i][m] * sd[i][k];
                                 T[3 * m + k] = dv * v;
                             }
-                        macc += rho * uu * dv;
+                        macc += uu * dv;
                     }
                     for (int k = 0; k < 9; ++k) Tq[c][f][k] = T[k];
                 }
             }
             __syncthreads();
-            // 5. per (node, mode): g[m] += sum_q T[m][k] dR/dx_k
+            // 5. per (node, pair): g[m] += sum_q T[m][k] dR/dx_k
 #pragma unroll
             for (int s = 0; s < GSL; ++s) {
                 const int x = t + 256 * s;
@@ -1789,28 +1811,28 @@ vib_grad_kernel(PatchArgs pa, double rho, VibModes vm, int64_t ebase,
         }
         if ((t & 3) == 0) mpart[(t >> 2) % VQC][(t >> 2) / VQC] = (t >> 2) / VQC < nf ? macc : 0.0;
         __syncthreads();
-        const int64_t eb = ebase + gi * nn;
 #pragma unroll
         for (int s = 0; s < GSL; ++s) {
             const int x = t + 256 * s;
-            if (x >= nn * VIB_MAXF) continue;
+            if (x >= nn * nf) continue;
             const int a = x % nn, f = x / nn;
 #pragma unroll
-            for (int m = 0; m < 3; ++m) eg[(eb + a) * (VIB_MAXF * 3) + 3 * f + m] = f < nf ? gr[s][m] : 0.0;
+            for (int m = 0; m < 3; ++m) eg[3 * (nf * (ebase + gi * nn + a) + f) + m] = gr[s][m];
         }
         if (t < VIB_MAXF) {
             double ms = 0.0;
             for (int c = 0; c < VQC; ++c) ms += mpart[c][t];
-            em[(mbase + gi) * VIB_MAXF + t] = ms;
+            em[gi * VIB_MAXF + t] = ms;
         }
     }
 }
 
-// Total mass of mode f over every element slot, in a fixed order (one block per mode).
-__global__ void __launch_bounds__(256) vib_mass_kernel(const double *em, int64_t nslot, double *mass) {
+// Total mass of pair f over the slots, in a fixed order (one block per pair).
+__global__ void __launch_bounds__(256) grad_mass_kernel(const double *em, int64_t nslot, double *mass) {
     __shared__ double sh[256];
     const int f = blockIdx.x;
     double v = 0.0;
+#pragma unroll 4
     for (int64_t i = threadIdx.x; i < nslot; i += 256) v += em[i * VIB_MAXF + f];
     sh[threadIdx.x] = v;
     __syncthreads();
@@ -1821,49 +1843,117 @@ __global__ void __launch_bounds__(256) vib_mass_kernel(const double *em, int64_t
     if (threadIdx.x == 0) mass[f] = sh[0];
 }
 
-// gradV(f0 + f, m, cp) = sum over the element-node entries of cp, in entry order, / mass[f]
-__global__ void __launch_bounds__(256) vib_gather_kernel(int32_t nb_cp, const int32_t *ptr, const int64_t *ent,
-                                                         const double *eg, const double *mass, VibModes vm,
-                                                         double *gradV) {
-    for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < 3 * (int64_t)nb_cp;
-         x += (int64_t)gridDim.x * blockDim.x) {
-        const int64_t cp = x / 3;
-        const int m = (int)(x % 3);
-        for (int f = 0; f < vm.nf; ++f) {
-            double s = 0.0;
-            for (int32_t j = ptr[cp]; j < ptr[cp + 1]; ++j) s += eg[ent[j] * (VIB_MAXF * 3) + 3 * f + m];
-            const double v = s * vm.scale;
-            gradV[(vm.f0 + f) + (int64_t)vm.nf_total * (m + 3 * cp)] = vm.normalize ? v / mass[f] : v;
-        }
+// out[k0 + f, m, cp] = scale times the sum over the element-node entries of cp, in entry order,
+// divided by mass[f] when mass is given; one thread per (cp, f, m), so that neighbouring threads
+// read an entry's pairs as one run (33x29x26 p=3, 4 modes: 62 us with the pairs in separate arrays
+// -> 28 us; the element kernel's stores, then in 24-byte runs, take 13 us more). GU entries are in
+// flight at once.
+__global__ void __launch_bounds__(256) grad_gather_kernel(int32_t nb_cp, const int32_t *__restrict__ ptr,
+                                                          const int32_t *__restrict__ ent,
+                                                          const double *__restrict__ eg, int32_t nf,
+                                                          const double *__restrict__ mass, double scale, int32_t k0,
+                                                          int32_t nk, double *__restrict__ out) {
+    constexpr int GU = 8;
+    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    const int row = 3 * nf;
+    if (x >= row * (int64_t)nb_cp) return;
+    const int32_t cp = (int32_t)(x / row);
+    const int fm = (int)(x - row * (int64_t)cp), f = fm / 3, m = fm - 3 * f;
+    const double *g = eg + fm;
+    double s = 0.0;
+    const int j1 = ptr[cp + 1];
+    for (int j = ptr[cp]; j < j1; j += GU) {
+        double v[GU];
+#pragma unroll
+        for (int u = 0; u < GU; ++u) v[u] = g[row * (int64_t)ent[min(j + u, j1 - 1)]];
+#pragma unroll
+        for (int u = 0; u < GU; ++u) s += j + u < j1 ? v[u] : 0.0;
+    }
+    s *= scale;
+    out[(k0 + f) + (int64_t)nk * (m + 3 * (int64_t)cp)] = mass ? s / mass[f] : s;
+}
+
+// the sum-factorised kernel takes max(p) + 1 Gauss points (all degrees the stiffness accepts);
+// other orders go to shape_grad_rt_kernel
+static bool grad_factorised(const PatchDev &pd) { return pd.tab_n >= 2 && pd.tab_n <= 5 && pd.ng == pd.tab_n; }
+
+// workgroups of the factorised kernel: a function of the element count only (each adds its
+// elements' masses), enough for several per CU
+template <int N, int Q>
+static unsigned grad_grid(int32_t n_active) {
+    constexpr int EPB = Grad<N, Q>::WPB * Grad<N, Q>::EPW;
+    return (unsigned)std::min<int64_t>((n_active + EPB - 1) / EPB, 3072);
+}
+
+static unsigned grad_slots(const PatchDev &pd) {
+    if (!grad_factorised(pd)) return (unsigned)pd.n_active;
+    switch (pd.tab_n) {
+    case 2: return grad_grid<2, 2>(pd.n_active);
+    case 3: return grad_grid<3, 3>(pd.n_active);
+    case 4: return grad_grid<4, 4>(pd.n_active);
+    default: return grad_grid<5, 5>(pd.n_active);
     }
 }
 
-template <int P, int NG, bool RT = false>
-static int launch_vib(yeti_asm *h, PatchDev &pd, const VibModes &vm, int64_t ebase, int64_t mbase, hipStream_t st) {
-    PatchArgs pa{};
-    pa.coords = h->coords.p;
-    pa.ien = pd.ien.p;
-    pa.weight = pd.weight.p;
-    pa.nijk = pd.nijk.p;
-    pa.U0 = pd.U[0].p;
-    pa.U1 = pd.U[1].p;
-    pa.U2 = pd.U[2].p;
-    pa.elems = pd.elems.p;
-    pa.n_active = pd.n_active;
-    pa.lam = pd.lam;
-    pa.mu = pd.mu;
-    gauss_legendre(RT ? pd.ng : NG, pa.g.x, pa.g.w);
-    VibDegrees dg{{pd.p[0], pd.p[1], pd.p[2]}, pd.ng};
-    const unsigned grid = (unsigned)std::min<int64_t>(pd.n_active, 1 << 20);
-    const double rho = vm.unit_density ? 1.0 : pd.rho;
-    hipLaunchKernelGGL((vib_grad_kernel<P, NG, RT>), dim3(grid), dim3(256), 0, st, pa, rho, vm, ebase, mbase,
-                       h->vib_eg.p, h->vib_em.p, dg);
+template <int N, int KIND>
+static void launch_grad(yeti_asm *h, PatchDev &pd, const GradFields &gf, int64_t ebase, int64_t mbase, hipStream_t st) {
+    GradArgs ga{};
+    ga.coords = h->coords.p;
+    ga.ien = pd.ien.p;
+    ga.weight = pd.weight.p;
+    ga.nijk = pd.nijk.p;
+    for (int d = 0; d < 3; ++d) {
+        ga.tab[d] = pd.tab[d].p;
+        ga.n[d] = pd.p[d] + 1;
+    }
+    ga.elems = pd.elems.p;
+    ga.n_active = pd.n_active;
+    ga.lam = pd.lam;
+    ga.mu = pd.mu;
+    gauss_legendre(N, ga.g.x, ga.g.w);
+    ga.f = gf;
+    ga.eg = h->vib_eg.p;
+    ga.ebase = ebase;
+    ga.em = h->vib_em.p + mbase * VIB_MAXF;
+    hipLaunchKernelGGL((shape_grad_kernel<N, N, KIND>), dim3(grad_grid<N, N>(pd.n_active)), dim3(64 * Grad<N, N>::WPB), 0,
+                       st, ga);
+}
+
+template <int KIND>
+static int launch_grad_kind(yeti_asm *h, PatchDev &pd, const GradFields &gf, int64_t ebase, int64_t mbase,
+                            hipStream_t st) {
+    if (grad_factorised(pd)) {
+        switch (pd.tab_n) {
+        case 2: launch_grad<2, KIND>(h, pd, gf, ebase, mbase, st); break;
+        case 3: launch_grad<3, KIND>(h, pd, gf, ebase, mbase, st); break;
+        case 4: launch_grad<4, KIND>(h, pd, gf, ebase, mbase, st); break;
+        default: launch_grad<5, KIND>(h, pd, gf, ebase, mbase, st); break;
+        }
+    } else {
+        PatchArgs pa{};
+        pa.coords = h->coords.p;
+        pa.ien = pd.ien.p;
+        pa.weight = pd.weight.p;
+        pa.nijk = pd.nijk.p;
+        pa.U0 = pd.U[0].p;
+        pa.U1 = pd.U[1].p;
+        pa.U2 = pd.U[2].p;
+        pa.elems = pd.elems.p;
+        pa.n_active = pd.n_active;
+        pa.lam = pd.lam;
+        pa.mu = pd.mu;
+        gauss_legendre(pd.ng, pa.g.x, pa.g.w);
+        GradDegrees dg{{pd.p[0], pd.p[1], pd.p[2]}, pd.ng};
+        const unsigned grid = (unsigned)std::min<int64_t>(pd.n_active, 1 << 20);
+        hipLaunchKernelGGL((shape_grad_rt_kernel<KIND>), dim3(grid), dim3(256), 0, st, pa, gf, dg, ebase, h->vib_eg.p,
+                           h->vib_em.p + mbase * VIB_MAXF);
+    }
     YETI_HIP(hipGetLastError());
     return 0;
 }
 
 // CP -> element-node entries of the active U1 elements (entry = patch base + gi nnode + a), in
-// patch, element and node order; buffers for the per-entry and per-element partials.
+// patch, element and node order; buffers for the per-entry partials and the masses.
 static int vib_setup(yeti_asm *h) {
     if (h->vib_nent >= 0) return 0;
     std::vector<int32_t> cnt(h->nb_cp + 1, 0);
@@ -1884,13 +1974,13 @@ static int vib_setup(yeti_asm *h) {
                 ++cnt[id];
             }
         nent += (int64_t)pd.n_active * pd.nnode;
-        nslot += pd.n_active;
+        nslot += grad_slots(pd);
     }
     if (nent > INT32_MAX) return set_error(YETI_ERR_SIZE_OVERFLOW, "vibration gradient: %lld element nodes", (long long)nent);
     std::vector<int32_t> ptr(h->nb_cp + 1, 0);
     for (int32_t c = 0; c < h->nb_cp; ++c) ptr[c + 1] = ptr[c] + cnt[c + 1];
     std::vector<int32_t> pos(ptr.begin(), ptr.end() - 1);
-    std::vector<int64_t> ent(std::max<int64_t>(nent, 1));
+    std::vector<int32_t> ent(std::max<int64_t>(nent, 1));
     int64_t base = 0;
     for (size_t k = 0; k < h->patches.size(); ++k) {
         PatchDev &pd = *h->patches[k];
@@ -1898,7 +1988,7 @@ static int vib_setup(yeti_asm *h) {
         for (int32_t gi = 0; gi < pd.n_active; ++gi)
             for (int a = 0; a < pd.nnode; ++a) {
                 const int32_t cp = ien_h[k][(size_t)pd.nnode * el_h[k][gi] + a] - 1;
-                ent[pos[cp]++] = base + (int64_t)gi * pd.nnode + a;
+                ent[pos[cp]++] = (int32_t)(base + (int64_t)gi * pd.nnode + a);
             }
         base += (int64_t)pd.n_active * pd.nnode;
     }
@@ -1912,90 +2002,62 @@ static int vib_setup(yeti_asm *h) {
     return 0;
 }
 
-static int run_vib_grad(yeti_asm *h, const double *vect, const double *vals, int32_t nf_total, double *gradV,
-                        hipStream_t st, double scale = 1.0, bool normalize = true, bool unit_density = false) {
+// Gradients of npair pairs (kind: shape_grad.hpp) over the active solid elements:
+// out[k, m, cp], (npair, 3, nb_cp) column-major, times scale, divided by the pair's mass when
+// normalize. f0: field 0 of GRAD_PAIRS; fk: the npair fields (npair, 3, nb_cp) column-major; vals
+// (host): eigenvalues, or null for 0. mass_out (device, one value per pair of the last launch), or
+// null.
+static int run_shape_grad(yeti_asm *h, GradKind kind, const double *f0, const double *fk, const double *vals,
+                          int32_t npair, double *out, double scale, bool normalize, double *mass_out, hipStream_t st) {
     for (auto *pd : h->patches) {
         if (!pd->u1 || pd->n_active == 0) continue;
-        const bool fixed = mfma_kernel_available(pd->p[0], pd->p[1], pd->p[2], pd->ng);
         const bool general = pd->p[0] >= 1 && pd->p[1] >= 1 && pd->p[2] >= 1 && pd->p[0] <= GEN_MAXP &&
                              pd->p[1] <= GEN_MAXP && pd->p[2] <= GEN_MAXP && pd->nnode <= GEN_MAXN && pd->ng >= 1 &&
                              pd->ng <= MAX_NG;
-        if (!fixed && !general)
-            return set_error(YETI_ERR_UNSUPPORTED_DEGREE, "vibration gradient: no kernel for degrees (%d,%d,%d), ng=%d",
+        if (!mfma_kernel_available(pd->p[0], pd->p[1], pd->p[2], pd->ng) && !general)
+            return set_error(YETI_ERR_UNSUPPORTED_DEGREE, "shape gradient: no kernel for degrees (%d,%d,%d), ng=%d",
                              pd->p[0], pd->p[1], pd->p[2], pd->ng);
     }
     int rc = vib_setup(h);
     if (rc) return rc;
-    for (int32_t f0 = 0; f0 < nf_total; f0 += VIB_MAXF) {
-        VibModes vm{};
-        vm.vect = vect;
-        vm.nf_total = nf_total;
-        vm.f0 = f0;
-        vm.nf = std::min<int32_t>(VIB_MAXF, nf_total - f0);
-        for (int f = 0; f < vm.nf; ++f) vm.vals[f] = vals[f0 + f];
-        vm.scale = scale;
-        vm.normalize = normalize ? 1 : 0;
-        vm.unit_density = unit_density ? 1 : 0;
+    for (int32_t k0 = 0; k0 < npair; k0 += VIB_MAXF) {
+        GradFields gf{};
+        gf.f0 = f0;
+        gf.fk = fk;
+        gf.nk = npair;
+        gf.k0 = k0;
+        gf.nf = std::min<int32_t>(VIB_MAXF, npair - k0);
+        for (int f = 0; f < gf.nf && vals; ++f) gf.vals[f] = vals[k0 + f];
         int64_t ebase = 0, mbase = 0;
         for (auto *pd : h->patches) {
             if (!pd->u1 || pd->n_active == 0) continue;
-            if (!mfma_kernel_available(pd->p[0], pd->p[1], pd->p[2], pd->ng))
-                rc = launch_vib<GEN_MAXP, MAX_NG, true>(h, *pd, vm, ebase, mbase, st);
-            else switch (pd->p[0] * 16 + pd->ng) {
-            case 1 * 16 + 2: rc = launch_vib<1, 2>(h, *pd, vm, ebase, mbase, st); break;
-            case 2 * 16 + 3: rc = launch_vib<2, 3>(h, *pd, vm, ebase, mbase, st); break;
-            case 3 * 16 + 4: rc = launch_vib<3, 4>(h, *pd, vm, ebase, mbase, st); break;
-            default: rc = launch_vib<4, 5>(h, *pd, vm, ebase, mbase, st); break;
-            }
+            gf.rho = pd->rho;
+            rc = kind == GRAD_MODES   ? launch_grad_kind<GRAD_MODES>(h, *pd, gf, ebase, mbase, st)
+                 : kind == GRAD_PAIRS ? launch_grad_kind<GRAD_PAIRS>(h, *pd, gf, ebase, mbase, st)
+                                      : launch_grad_kind<GRAD_VOLUME>(h, *pd, gf, ebase, mbase, st);
             if (rc) return rc;
             ebase += (int64_t)pd->n_active * pd->nnode;
-            mbase += pd->n_active;
+            mbase += grad_slots(*pd);
         }
-        if (h->vib_nslot > 0) {
-            hipLaunchKernelGGL(vib_mass_kernel, dim3(vm.nf), dim3(256), 0, st, (const double *)h->vib_em.p, h->vib_nslot,
-                               h->vib_mass.p);
-        } else {   // no active element: zero mass, as the reference's empty sum
-            hipLaunchKernelGGL(fill_zero_kernel, dim3(1), dim3(256), 0, st, h->vib_mass.p, (int32_t *)nullptr,
-                               (int32_t *)nullptr, (int64_t)VIB_MAXF);
+        double *mass = mass_out ? mass_out : h->vib_mass.p;
+        if (normalize || mass_out) {   // no active element: zero mass, as the reference's empty sum
+            hipLaunchKernelGGL(grad_mass_kernel, dim3(gf.nf), dim3(256), 0, st, (const double *)h->vib_em.p, h->vib_nslot,
+                               mass);
+            YETI_HIP(hipGetLastError());
         }
-        YETI_HIP(hipGetLastError());
-        const int blocks = (int)std::max<int64_t>(1, std::min<int64_t>((3 * (int64_t)h->nb_cp + 255) / 256, 65536));
-        hipLaunchKernelGGL(vib_gather_kernel, dim3(blocks), dim3(256), 0, st, h->nb_cp, (const int32_t *)h->vib_ptr.p,
-                           (const int64_t *)h->vib_ent.p, (const double *)h->vib_eg.p, (const double *)h->vib_mass.p,
-                           vm, gradV);
+        const unsigned blocks = (unsigned)((3 * gf.nf * (int64_t)h->nb_cp + 255) / 256);
+        hipLaunchKernelGGL(grad_gather_kernel, dim3(blocks), dim3(256), 0, st, h->nb_cp, (const int32_t *)h->vib_ptr.p,
+                           (const int32_t *)h->vib_ent.p, (const double *)h->vib_eg.p, gf.nf,
+                           normalize ? (const double *)mass : (const double *)nullptr, scale, k0, npair, out);
         YETI_HIP(hipGetLastError());
     }
     return 0;
 }
 
-// -d(u^T K u)/dX (3 per CP, COORDS3D order) over the active solid elements: the gradient kernel
-// with eigenvalue 0 (no mass term), the sums scaled by -1 and not normalised. u is dof-interleaved
-// (3 cp + c), which is the (1, 3, nb_cp) column-major layout of one mode.
+// -d(u^T K u)/dX (3 per CP, COORDS3D order): eigenvalue 0, the sums scaled by -1 and not
+// normalised. u is dof-interleaved (3 cp + c), the (1, 3, nb_cp) column-major layout of one field.
 static int run_strain_energy_grad(yeti_asm *h, const double *u, double *g, hipStream_t st) {
-    const double zero = 0.0;
-    return run_vib_grad(h, u, &zero, 1, g, st, -1.0, false);
-}
-
-// u = e_x at every control point (a rigid translation)
-__global__ void translation_kernel(double *u, int64_t n3) {
-    const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n3) u[i] = i % 3 == 0 ? 1.0 : 0.0;
-}
-
-// Volume of the active solid elements and its derivative dV/dX (3 per CP): the gradient kernel
-// for the translation u = e_x with density 1 and eigenvalue -1. Then du/dx = 0, |u| = 1, the
-// per-point tensor is w|J| I, so the CP sums are sum_q w|J| dR_a/dx_m = dV/dX_am, and the
-// "mass" u^T M u is sum_q w|J| = V. vol (device, 1 value) and g (device, 3 nb_cp).
-static int run_volume_grad(yeti_asm *h, double *vol, double *g, hipStream_t st) {
-    const int64_t n3 = 3 * (int64_t)h->nb_cp;
-    if (!h->vol_u.p) YETI_HIP(h->vol_u.alloc((size_t)std::max<int64_t>(n3, 1)));
-    hipLaunchKernelGGL(translation_kernel, dim3((unsigned)((n3 + 255) / 256)), dim3(256), 0, st, h->vol_u.p, n3);
-    YETI_HIP(hipGetLastError());
-    const double eig = -1.0;
-    int rc = run_vib_grad(h, h->vol_u.p, &eig, 1, g, st, 1.0, false, true);
-    if (rc) return rc;
-    YETI_HIP(hipMemcpyAsync(vol, h->vib_mass.p, sizeof(double), hipMemcpyDeviceToDevice, st));
-    return 0;
+    return run_shape_grad(h, GRAD_MODES, nullptr, u, nullptr, 1, g, -1.0, false, nullptr, st);
 }
 
 // u^T F shape derivative of the face and body loads: g = 2 u^T dF/dX (3 per CP), gathered like F.
@@ -2043,46 +2105,6 @@ static int run_load_grad(yeti_asm *h, const double *u, double *g, hipStream_t st
 // ---- gradLinElastWork_AN: internal and external work gradients for given SOL and ADJ --------
 // Fields f of an (nf, 3, nb_cp) column-major array sit at f + nf (3 cp + d).
 
-// sums[f] = sum over (d, cp) of V[f, d, cp]^2, one block per field, fixed order (deterministic)
-__global__ void __launch_bounds__(256) field_sumsq_kernel(const double *V, int32_t nf, int64_t n3, double *sums) {
-    const int f = blockIdx.x;
-    double s = 0.0;
-    for (int64_t j = threadIdx.x; j < n3; j += blockDim.x) {
-        const double v = V[f + (int64_t)nf * j];
-        s += v * v;
-    }
-    __shared__ double red[256];
-    red[threadIdx.x] = s;
-    __syncthreads();
-    for (int o = 128; o > 0; o >>= 1) {
-        if ((int)threadIdx.x < o) red[threadIdx.x] += red[threadIdx.x + o];
-        __syncthreads();
-    }
-    if (threadIdx.x == 0) sums[f] = red[0];
-}
-
-// V[2k] = u + s_k a_k, V[2k + 1] = u - s_k a_k (fields of an (2 nadj, 3, nb_cp) array)
-__global__ void polar_fields_kernel(const double *u, const double *adj, int32_t nadj, int64_t n3, const double *scale,
-                                    double *V) {
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= n3 * nadj) return;
-    const int64_t j = x / nadj;
-    const int k = (int)(x % nadj);
-    const double a = scale[k] * adj[k + (int64_t)nadj * j];
-    V[2 * k + (int64_t)(2 * nadj) * j] = u[j] + a;
-    V[2 * k + 1 + (int64_t)(2 * nadj) * j] = u[j] - a;
-}
-
-// out[k, j] = (G[2k, j] - G[2k + 1, j]) / (4 s_k): the polarisation of the quadratic form
-__global__ void polar_combine_kernel(const double *G, int32_t nadj, int64_t n3, const double *scale, double *out) {
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    if (x >= n3 * nadj) return;
-    const int64_t j = x / nadj;
-    const int k = (int)(x % nadj);
-    out[k + (int64_t)nadj * j] =
-        (G[2 * k + (int64_t)(2 * nadj) * j] - G[2 * k + 1 + (int64_t)(2 * nadj) * j]) / (4.0 * scale[k]);
-}
-
 // a[j] = ADJ[k, j] and back: out[k, j] = c g[j]
 __global__ void field_extract_kernel(const double *adj, int32_t nadj, int32_t k, int64_t n3, double *a) {
     const int64_t j = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -2094,42 +2116,15 @@ __global__ void field_insert_kernel(const double *g, double c, int32_t nadj, int
 }
 
 // gradWint[k] = -ADJ_k^T (dK/dX) SOL and gradWext[k] = ADJ_k^T (dF/dX) over the active solid
-// elements (gradtotalwork_fullAN.f90:17-300). The internal term is bilinear and symmetric, and
-// the gradient kernel gives the quadratic form q(v) = -v^T (dK/dX) v, so
-//   -a^T (dK/dX) u = (q(u + s a) - q(u - s a)) / (4 s),
-// with s = |u| / |a| so that both fields have the norm of u (no cancellation beyond rounding);
-// the 2 nadj fields run through the kernel together (its field-independent work is shared).
+// elements (gradtotalwork_fullAN.f90:17-300): the pairs (SOL, ADJ_k), VIB_MAXF per launch (the
+// geometry and the state are evaluated once for them).
 static int run_grad_lin_elast_work(yeti_asm *h, const double *sol, const double *adj, int32_t nadj, bool wint,
                                    bool wext, double *gint, double *gext, hipStream_t st) {
     const int64_t n3 = 3 * (int64_t)h->nb_cp;
     const unsigned blk = (unsigned)((n3 * nadj + 255) / 256), blk1 = (unsigned)((n3 + 255) / 256);
-    if (h->gw_sums.n < (size_t)(2 * nadj + 1)) YETI_HIP(h->gw_sums.alloc(2 * (size_t)nadj + 1));
     if (wint) {
-        if (h->gw_fields.n < (size_t)(2 * nadj * n3)) {
-            YETI_HIP(h->gw_fields.alloc((size_t)(2 * nadj * n3)));
-            YETI_HIP(h->gw_grads.alloc((size_t)(2 * nadj * n3)));
-        }
-        double *sums = h->gw_sums.p, *scale = h->gw_sums.p + nadj + 1;
-        hipLaunchKernelGGL(field_sumsq_kernel, dim3(1), dim3(256), 0, st, sol, 1, n3, sums);
-        hipLaunchKernelGGL(field_sumsq_kernel, dim3(nadj), dim3(256), 0, st, adj, nadj, n3, sums + 1);
-        YETI_HIP(hipGetLastError());
-        std::vector<double> hs(nadj + 1), sc(nadj);
-        YETI_HIP(hipMemcpyAsync(hs.data(), sums, (nadj + 1) * sizeof(double), hipMemcpyDeviceToHost, st));
-        YETI_HIP(hipStreamSynchronize(st));
-        for (int k = 0; k < nadj; ++k)
-            sc[k] = (hs[0] > 0.0 && hs[k + 1] > 0.0) ? std::sqrt(hs[0] / hs[k + 1]) : 1.0;
-        YETI_HIP(hipMemcpyAsync(scale, sc.data(), nadj * sizeof(double), hipMemcpyHostToDevice, st));
-        hipLaunchKernelGGL(polar_fields_kernel, dim3(blk), dim3(256), 0, st, sol, adj, nadj, n3, (const double *)scale,
-                           h->gw_fields.p);
-        YETI_HIP(hipGetLastError());
-        std::vector<double> zeros(2 * nadj, 0.0);
-        int rc = run_vib_grad(h, h->gw_fields.p, zeros.data(), 2 * nadj, h->gw_grads.p, st, -1.0, false);
+        int rc = run_shape_grad(h, GRAD_PAIRS, sol, adj, nullptr, nadj, gint, -1.0, false, nullptr, st);
         if (rc) return rc;
-        hipLaunchKernelGGL(polar_combine_kernel, dim3(blk), dim3(256), 0, st, (const double *)h->gw_grads.p, nadj, n3,
-                           (const double *)scale, gint);
-        YETI_HIP(hipGetLastError());
-        // the host copy of the scales must outlive the copy above
-        YETI_HIP(hipStreamSynchronize(st));
     } else {
         hipLaunchKernelGGL(fill_zero_kernel, dim3(blk), dim3(256), 0, st, gint, (int32_t *)nullptr, (int32_t *)nullptr,
                            n3 * nadj);
@@ -2139,6 +2134,9 @@ static int run_grad_lin_elast_work(yeti_asm *h, const double *sol, const double 
         if (!h->ref_infos_ok)
             return set_error(YETI_ERR_INVALID_ARGUMENT,
                              "load_additionalInfos holds fewer than 6 values per centrifugal load");
+        wext = h->any_centrifugal;   // without one the term is zero
+    }
+    if (wext) {
         if (h->gw_vec.n < (size_t)n3) {
             YETI_HIP(h->gw_vec.alloc(n3));
             YETI_HIP(h->gw_vec2.alloc(n3));
@@ -2301,8 +2299,14 @@ static int create(const yeti_system_inputs *in, int layout, yeti_asm **out) {
         pd->u1 = pd->u1 || u0;
         pd->n_active = (int32_t)act.size();
         hipError_t e1 = hipSuccess;
+        pd->tab_n = act.empty() ? 0 : std::max(std::max(pd->p[0], pd->p[1]), pd->p[2]) + 1;
         for (int d = 0; d < 3 && e1 == hipSuccess; ++d) {
             e1 = pd->U[d].upload(in->Ukv + kv, nkv[d]);
+            if (e1 == hipSuccess && pd->tab_n == pd->ng) {
+                std::vector<double> tab;
+                basis_table(pd->p[d], in->Ukv + kv, nkv[d], pd->tab_n, tab);
+                e1 = pd->tab[d].upload(tab.data(), tab.size());
+            }
             kv += nkv[d];
         }
         if (e1 == hipSuccess) e1 = pd->ien.upload(in->IEN + ieoff, (size_t)pd->nnode * pd->nelem);
@@ -2381,6 +2385,7 @@ static int create(const yeti_system_inputs *in, int layout, yeti_asm **out) {
     int64_t n101 = 0;
     for (int il = 0; il < in->nb_load; ++il)
         if (in->JDLType[il] == 101) add_off_ref[il] = (int32_t)(6 * n101++);
+    h->any_centrifugal = n101 > 0;
     h->ref_infos_ok = 6 * n101 <= std::max<int64_t>(0, in->len_load_additionalInfos);
     if (in->nb_load > 0 && add_off[in->nb_load] > std::max<int64_t>(0, in->len_load_additionalInfos))
         return fail(set_error(YETI_ERR_INVALID_ARGUMENT, "load_additionalInfos holds %lld values, the loads name %d",
@@ -2507,7 +2512,8 @@ int32_t yeti_asm_run_vib_grad(yeti_asm *h, const double *vect, const double *val
                               void *stream) {
     if (!h || !vect || !vals || !gradV || nb_frq < 1)
         return yeti::set_error(YETI_ERR_INVALID_ARGUMENT, "null argument or nb_frq < 1");
-    return yeti::run_vib_grad(h, vect, vals, nb_frq, gradV, (hipStream_t)stream);
+    return yeti::run_shape_grad(h, yeti::GRAD_MODES, nullptr, vect, vals, nb_frq, gradV, 1.0, true, nullptr,
+                                (hipStream_t)stream);
 }
 
 int32_t yeti_asm_strain_energy_grad(yeti_asm *h, const double *u, double *g, void *stream) {
@@ -2517,7 +2523,8 @@ int32_t yeti_asm_strain_energy_grad(yeti_asm *h, const double *u, double *g, voi
 
 int32_t yeti_asm_volume_grad(yeti_asm *h, double *vol, double *g, void *stream) {
     if (!h || !vol || !g) return yeti::set_error(YETI_ERR_INVALID_ARGUMENT, "null argument");
-    return yeti::run_volume_grad(h, vol, g, (hipStream_t)stream);
+    return yeti::run_shape_grad(h, yeti::GRAD_VOLUME, nullptr, nullptr, nullptr, 1, g, 1.0, false, vol,
+                                (hipStream_t)stream);
 }
 
 int32_t yeti_grad_lin_elast_work(yeti_asm *h, const double *SOL, const double *ADJ, int32_t nadj, int32_t computeWint,
