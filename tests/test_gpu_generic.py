@@ -177,3 +177,43 @@ def test_gpu_general_degrees_postprocessing_match_oracle(name):
     u = evaldisp_points(1, xi, sol.T, **kw)
     uo = O.oracle_evaldisp(1, xi, sol.T, **kw)
     assert np.abs(u - uo).max() <= 1e-13 * np.abs(uo).max()
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("deg,nel,ng", [((1, 1, 1), (3, 3, 1), 2), ((2, 2, 2), (5, 1, 2), 3), ((4, 2, 1), (2, 2, 2), 5),
+                                        ((3, 3, 2), (2, 1, 2), 4), ((3, 4, 2), (1, 2, 1), 5), ((3, 3, 3), (1, 1, 2), 9)])
+def test_gpu_general_kernel_tiles_and_offsets(deg, nel, ng):
+    """elem_general at 8 to 64 nodes (one to four node tiles, full and partly filled; above 32
+    nodes the entries leave in several rounds), 8 to 729 points (whole and partial chunks),
+    elements whose COO range starts at odd entries and at every inactive-element offset, and
+    outputs at an odd address: stiffness and mass against the oracle, indices bit-exact, values
+    within 1e-12 of their maximum."""
+    import torch
+    from perf.cases import _model
+    from yeti_amd.assembly import Assembler
+    print("[case] general kernel degrees %s ng=%d" % (deg, ng), flush=True)
+    case = dict(n0=nel[0], n1=nel[1], n2=nel[2], p0=deg[0], p1=deg[1], p2=deg[2], ng=ng)
+    d = _model(case, 3)
+    d["activeElement"] = d["activeElement"].copy()
+    d["activeElement"][1] = 0
+    Ko, ro, co, _ = O.oracle_sys_linmat([], kwargs={k.lower(): v for k, v in d.items()})
+    Mo = O.oracle_mass_coo(d)[0]
+    asm = Assembler(d)
+    try:
+        n = asm.nb_data
+        for off in (0, 1):
+            K = torch.zeros(n + 2, dtype=torch.float64, device="cuda")[off:]
+            r, c = (torch.zeros(n + 4, dtype=torch.int32, device="cuda")[k + off:] for k in (0, 1))
+            asm.run_matrix(K, r, c)
+            assert np.array_equal(r[:n].cpu().numpy(), ro[:n]) and np.array_equal(c[:n].cpu().numpy(), co[:n])
+            assert np.abs(K[:n].cpu().numpy() - Ko[:n]).max() <= 1e-12 * np.abs(Ko).max()
+            assert float(K[n:].abs().max()) == 0.0
+            V = torch.zeros(n + 1, dtype=torch.float64, device="cuda")
+            asm.run_values(V)
+            assert torch.equal(V[:n], K[:n])
+            r.zero_()
+            M = asm.run_mass(K, r, c)[0]
+            assert np.array_equal(r[:n].cpu().numpy(), ro[:n]) and np.array_equal(c[:n].cpu().numpy(), co[:n])
+            assert np.abs(M[:n].cpu().numpy() - Mo[:n]).max() <= 1e-12 * np.abs(Mo).max()
+    finally:
+        asm.close()
