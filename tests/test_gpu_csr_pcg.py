@@ -58,6 +58,31 @@ def test_csr_matches_scipy(gpu, nel, p):
     _check_case(bp.args, "csr box %s p=%d" % (nel, p))
 
 
+@pytest.mark.parametrize("nel,p,relabel", [((9, 8, 7), 1, False), ((9, 8, 7), 1, True), ((6, 5, 5), 2, False),
+                                           ((6, 5, 5), 2, True), ((3, 2, 1), 2, True), ((3, 4, 3), 3, True),
+                                           ((3, 4, 3), 3, False), ((3, 2, 2), 4, False)])
+def test_csr_values_by_rows_and_by_blocks(gpu, nel, p, relabel):
+    """The ways the values are gathered: whole element rows (elements numbered against their
+    control points, rows long enough, one or two slots per lane), and block by block (short rows,
+    16 to 64 lanes each; control points numbered at random), with inactive elements."""
+    a = dict(make_box_patch(nel=nel, p=p, seed=4 + p).args)
+    a["activeElement"] = a["activeElement"].copy()
+    a["activeElement"][[0, -1]] = 0
+    if relabel:
+        ncp = int(a["nb_cp"])
+        new = np.random.default_rng(p).permutation(ncp)          # old id -> new id, 0-based
+        X = np.empty_like(a["COORDS3D"])
+        X[:, new] = a["COORDS3D"]
+        a["COORDS3D"] = np.asfortranarray(X)
+        a["IEN"] = (new[a["IEN"] - 1] + 1).astype(np.int32)
+        a["bc_target"] = (new[a["bc_target"] - 1] + 1).astype(np.int32)
+        free = a["ind_dof_free"][:a["nb_dof_free"]].astype(np.int64) - 1
+        ind = np.zeros_like(a["ind_dof_free"])
+        ind[:free.size] = np.sort(3 * new[free // 3] + free % 3) + 1
+        a["ind_dof_free"] = ind
+    _check_case(a, "csr %s p=%d relabel=%s" % (nel, p, relabel))
+
+
 def test_csr_multipatch(gpu):
     m = concat_patches(make_box_patch(nel=(3, 2, 2), p=2, seed=1), make_box_patch(nel=(2, 2, 2), p=3, seed=2))
     _check_case(m, "csr two patches")

@@ -6,15 +6,16 @@
 //
 // Pattern (once, from the resident connectivity): CP -> (element, local node) incidence,
 // sorted by element; per CP row the sorted set of CPs sharing an element (3x3 block pattern);
-// per block the list of element contributions in ascending element order. Values (every
-// assembly): one thread per block sums its contributions read from the COO values in that fixed
-// order -- deterministic, no floating-point atomics. Scalar CSR: dof row 3 I + k holds, for each
+// per block J >= I the list of element contributions in ascending element order. Values (every
+// assembly): one thread per such block sums its contributions read from the COO values in that fixed
+// order -- deterministic, no floating-point atomics -- and writes the block and its transpose. Scalar CSR: dof row 3 I + k holds, for each
 // block column J of CP row I (ascending), the columns 3 J, 3 J + 1, 3 J + 2: scipy's canonical
 // layout of the structural pattern.
 #include <algorithm>
 #include <vector>
 
 #include "common.hpp"
+#include "copy_out.hpp"
 
 namespace yeti {
 // declared in assembly.hip
@@ -35,7 +36,16 @@ struct yeti_csr {
     int64_t nblocks = 0;                 // 3x3 blocks
     yeti::DevBuf<int64_t> bptr;          // [nb_cp + 1]
     yeti::DevBuf<int32_t> bcol;          // [nblocks]
-    yeti::DevBuf<int64_t> cptr;          // [nblocks + 1] contribution offsets
+    yeti::DevBuf<int32_t> bdiag;         // [nb_cp] place of the diagonal block in its row (the row's length: none)
+    yeti::DevBuf<uint16_t> mirror;       // [nblocks] block (I, J), J > I: place of block (J, I) in row J
+    // values by element rows (row_values_kernel), when upper > 0:
+    int32_t upper = 0;                   // most blocks J >= I of a row
+    int32_t sstride = 0;                 // slots per incidence
+    yeti::DevBuf<int64_t> iptr;          // [nb_cp + 1] incidences of each CP
+    yeti::DevBuf<int64_t> irow;          // (COO position of the element's row of a << 10) | a
+    yeti::DevBuf<uint16_t> slots;        // [incidence][b]: place of block (I, J_b) after the diagonal, b <= a
+    // values by blocks (csr_values_kernel) otherwise:
+    yeti::DevBuf<int64_t> cptr;          // [nblocks + 1] contribution offsets (blocks J >= I)
     yeti::DevBuf<int64_t> contrib;       // (COO position << 2) | kind
     yeti::DevBuf<int64_t> rowptr;        // scalar CSR [3 nb_cp + 1]
     yeti::DevBuf<int32_t> colind;        // scalar CSR [9 nblocks]
@@ -218,7 +228,7 @@ __global__ void __launch_bounds__(256) row_pattern_kernel(int32_t nb_cp, const i
     }
 }
 
-// Per row: count (pass 1) or write (pass 2) the contributions of each block, in element order.
+// Per row: count (pass 1) or write (pass 2) the contributions of each block J >= I, in element order.
 // kind 0: block (a, b) stored as is (a < b); 1: stored as (b, a) (a > b, transpose);
 // 2: diagonal block (a == b), stored as its 6 upper entries with the diagonal halved.
 template <bool FILL>
@@ -242,6 +252,7 @@ __global__ void __launch_bounds__(64) contrib_kernel(int32_t nb_cp, const int64_
         const int32_t *ie = pi.ien[patch] + (int64_t)nn * e;
         for (int b = lane; b < nn; b += 64) {
             int32_t J = ie[b] - 1;
+            if (J < row) continue;
             int lo = 0, hi = nb - 1;       // binary search of J among the row's sorted columns
             while (lo < hi) {
                 int mid = (lo + hi) >> 1;
@@ -261,6 +272,27 @@ __global__ void __launch_bounds__(64) contrib_kernel(int32_t nb_cp, const int64_
     }
     if (!FILL)
         for (int i = lane; i < nb; i += 64) bcount[b0 + i] = cur[i];
+}
+
+// The diagonal block's place in each row, and for every block above it the place of its transpose.
+__global__ void __launch_bounds__(256) mirror_kernel(int32_t nb_cp, const int64_t *__restrict__ bptr,
+                                                     const int32_t *__restrict__ bcol, int32_t *__restrict__ bdiag,
+                                                     uint16_t *__restrict__ mirror) {
+    const int64_t I = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (I >= nb_cp) return;
+    const int lane = threadIdx.x & 63;
+    auto place = [&](int64_t row, int32_t col) {   // first column >= col
+        int lo = 0, hi = (int)(bptr[row + 1] - bptr[row]);
+        const int32_t *c = bcol + bptr[row];
+        while (lo < hi) {
+            const int mid = (lo + hi) >> 1;
+            if (c[mid] < col) lo = mid + 1; else hi = mid;
+        }
+        return lo;
+    };
+    const int jd = place(I, (int32_t)I), nb = (int)(bptr[I + 1] - bptr[I]);
+    if (lane == 0) bdiag[I] = jd;
+    for (int j = jd + lane; j < nb; j += 64) mirror[bptr[I] + j] = (uint16_t)place(bcol[bptr[I] + j], (int32_t)I);
 }
 
 __global__ void scalar_pattern_kernel(int32_t nb_cp, const int64_t *bptr, const int32_t *bcol,
@@ -286,51 +318,237 @@ __global__ void scalar_pattern_kernel(int32_t nb_cp, const int64_t *bptr, const 
 }
 
 // ---- values ------------------------------------------------------------------------------
-__global__ void csr_values_kernel(int32_t nb_cp, const int64_t *bptr, const int64_t *cptr,
-                                  const int64_t *contrib, const double *__restrict__ Kdata,
-                                  double *__restrict__ vals) {
-    // one thread per block; blocks of a row are consecutive threads
-    int64_t blk = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
-    int64_t nblocks = bptr[nb_cp];
-    if (blk >= nblocks) return;
-    // row of this block: binary search in bptr
-    int lo = 0, hi = nb_cp - 1;
-    while (lo < hi) {
-        int mid = (lo + hi + 1) >> 1;
-        if (bptr[mid] <= blk) lo = mid; else hi = mid - 1;
-    }
-    const int I = lo;
+// LPR lanes per CP row I, each on a block J >= I (its contributions summed in element order), written
+// as block (I, J) and, transposed, as (J, I): each COO value is read once. Local nodes are numbered
+// against the CPs, so a block above the diagonal mostly holds a > b and lies in the element's row of a:
+// its neighbours' contributions are next to it and the lanes read whole cache lines, where the blocks
+// below the diagonal would take 72 bytes out of every line pair. A contribution is read in five loads,
+// UC of them in flight. Each XCD takes one run of rows, so that the transposed blocks of neighbouring
+// rows meet in its L2. 45x40x33 p = 3: 5.35 ms (21.5 GB fetched), against 7.72 ms with one thread for
+// every block, found by binary search; 100x60x60 p = 1, which row_values_kernel does not take,
+// 0.98 -> 0.85 ms with the product.
+typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
+
+template <int LPR>
+__global__ void __launch_bounds__(256) csr_values_kernel(int32_t nb_cp, const int64_t *__restrict__ bptr,
+                                                         const int32_t *__restrict__ bcol,
+                                                         const int32_t *__restrict__ bdiag,
+                                                         const uint16_t *__restrict__ mirror,
+                                                         const int64_t *__restrict__ cptr,
+                                                         const int64_t *__restrict__ contrib,
+                                                         const double *__restrict__ Kdata,
+                                                         double *__restrict__ vals) {
+    constexpr int UC = 2;
+    constexpr int RPB = 256 / LPR;   // rows per workgroup
+    const int lane = threadIdx.x % LPR;
+    const int64_t I = xcd_element(blockIdx.x, ((int64_t)nb_cp + RPB - 1) / RPB) * RPB + threadIdx.x / LPR;
+    if (I >= nb_cp) return;
     const int64_t b0 = bptr[I];
     const int nb = (int)(bptr[I + 1] - b0);
-    const int j = (int)(blk - b0);
-    double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};   // v[k][l] = v[3k + l]
-    for (int64_t c = cptr[blk]; c < cptr[blk + 1]; ++c) {
-        int64_t code = contrib[c];
-        int kind = (int)(code & 3);
-        const double *s = Kdata + (code >> 2);
-        if (kind == 0) {            // stored (k, l) at s[k + 3 l]
+    for (int j = bdiag[I] + lane; j < nb; j += LPR) {
+        double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};   // v[k][l] = v[3k + l]
+        const int32_t J = bcol[b0 + j];
+        const int jm = mirror[b0 + j];
+        const int64_t c1 = cptr[b0 + j + 1];
+        for (int64_t c = cptr[b0 + j]; c < c1; c += UC) {
+            double s[UC][9];
+            int kind[UC];
+#pragma unroll
+            for (int u = 0; u < UC; ++u) {
+                const int64_t code = contrib[min(c + u, c1 - 1)];
+                kind[u] = c + u < c1 ? (int)(code & 3) : 3;
+                const double *p = Kdata + (code >> 2);
+                f64x2u t[4] = {};
+                t[0] = *reinterpret_cast<const f64x2u *>(p);
+                t[1] = *reinterpret_cast<const f64x2u *>(p + 2);
+                t[2] = *reinterpret_cast<const f64x2u *>(p + 4);
+                s[u][8] = 0.0;
+                if ((code & 3) != 2) {   // a diagonal block has six entries
+                    t[3] = *reinterpret_cast<const f64x2u *>(p + 6);
+                    s[u][8] = p[8];
+                }
+#pragma unroll
+                for (int x = 0; x < 8; ++x) s[u][x] = t[x / 2][x % 2];
+            }
+#pragma unroll
+            for (int u = 0; u < UC; ++u) {
+                const double *q = s[u];
+                if (kind[u] < 2) {   // stored (k, l) at q[k + 3 l]; kind 1: the transpose of the stored block
+                    const bool tr = kind[u] == 1;
+#pragma unroll
+                    for (int k = 0; k < 3; ++k)
+#pragma unroll
+                        for (int l = 0; l < 3; ++l) v[3 * k + l] += tr ? q[l + 3 * k] : q[k + 3 * l];
+                } else if (kind[u] == 2) {   // diagonal block: side + side^T, (0,0) (0,1) (1,1) (0,2) (1,2) (2,2)
+                    v[0] += 2.0 * q[0]; v[4] += 2.0 * q[2]; v[8] += 2.0 * q[5];
+                    v[1] += q[1]; v[3] += q[1];
+                    v[2] += q[3]; v[6] += q[3];
+                    v[5] += q[4]; v[7] += q[4];
+                }
+            }
+        }
+        double *o = vals + 9 * b0 + 3 * j;
+#pragma unroll
+        for (int k = 0; k < 3; ++k)
+#pragma unroll
+            for (int l = 0; l < 3; ++l) o[3LL * k * nb + l] = v[3 * k + l];
+        if (J != I) {
+            const int64_t m0 = bptr[J];
+            const int mb = (int)(bptr[J + 1] - m0);
+            o = vals + 9 * m0 + 3 * jm;
 #pragma unroll
             for (int k = 0; k < 3; ++k)
 #pragma unroll
-                for (int l = 0; l < 3; ++l) v[3 * k + l] += s[k + 3 * l];
-        } else if (kind == 1) {     // transpose of the stored block
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-#pragma unroll
-                for (int l = 0; l < 3; ++l) v[3 * k + l] += s[l + 3 * k];
-        } else {                    // diagonal block: side + side^T
-            const double d00 = s[0], d01 = s[1], d11 = s[2], d02 = s[3], d12 = s[4], d22 = s[5];
-            v[0] += 2.0 * d00; v[4] += 2.0 * d11; v[8] += 2.0 * d22;
-            v[1] += d01; v[3] += d01;
-            v[2] += d02; v[6] += d02;
-            v[5] += d12; v[7] += d12;
+                for (int l = 0; l < 3; ++l) o[3LL * k * mb + l] = v[3 * l + k];
         }
     }
-    const int64_t r0 = 9 * b0;
+}
+
+// Values by element rows. Local nodes are numbered against the CPs (b < a holds CPs J_b > I_a), so the
+// 9 a + 6 COO entries of an element's row a are exactly its contributions to the blocks J >= I of the
+// CP I of a: one wave per CP row streams those runs whole, element after element, into the row's
+// blocks in LDS (entry x of a run goes to entry x mod 9 of block x / 9, through the incidence's slots).
+// Every address is added to by one wave in a fixed order. Then the row is written with consecutive
+// lanes on consecutive values, and its transposes. Loads run one group of RG ahead.
+constexpr int ROW_WAVES = 2;   // rows per workgroup (LDS: 12 waves per CU at p = 3)
+
+template <int NSL>   // slots per lane: 1 up to 64 nodes per element, 2 up to 128
+__global__ void __launch_bounds__(64 * ROW_WAVES)
+row_values_kernel(int32_t nb_cp, int32_t upper, int32_t sstride, const int64_t *__restrict__ bptr,
+                  const int32_t *__restrict__ bcol, const int32_t *__restrict__ bdiag,
+                  const uint16_t *__restrict__ mirror, const int64_t *__restrict__ iptr,
+                  const int64_t *__restrict__ irow, const uint16_t *__restrict__ slots,
+                  const double *__restrict__ Kdata, double *__restrict__ vals) {
+    constexpr int RG = 5;
+    extern __shared__ double racc[];
+    const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    double *acc = racc + wv * 9 * upper;
+    const int64_t I = xcd_element(blockIdx.x, ((int64_t)nb_cp + ROW_WAVES - 1) / ROW_WAVES) * ROW_WAVES + wv;
+    if (I >= nb_cp) return;   // waves of a workgroup share nothing
+    const int64_t b0 = bptr[I];
+    const int nb = (int)(bptr[I + 1] - b0), jd = bdiag[I], nu = nb - jd;
+    for (int x = lane; x < 9 * nu; x += 64) acc[x] = 0.0;
+    const int64_t k1 = iptr[I + 1];
+    int64_t k = iptr[I], code = k < k1 ? irow[k] : 0, next = k + 1 < k1 ? irow[k + 1] : 0;
+    int x0 = 0;
+    double v[RG];
+    uint16_t sl[NSL] = {};   // slots of b = lane, lane + 64
+    auto fetch = [&](int64_t kk, int64_t cd, int xx, double (&o)[RG], uint16_t (&so)[NSL]) {
+        const int a = (int)(cd & 1023), len = 9 * a + 6;
+        const double *run = Kdata + (cd >> 10);
 #pragma unroll
-    for (int k = 0; k < 3; ++k)
+        for (int u = 0; u < RG; ++u) {
+            const int x = xx + lane + 64 * u;
+            o[u] = x < len ? run[x] : 0.0;
+        }
+        if (xx == 0) {
+            const uint16_t *sp = slots + kk * sstride;
 #pragma unroll
-        for (int l = 0; l < 3; ++l) vals[r0 + 3LL * k * nb + 3 * j + l] = v[3 * k + l];
+            for (int h = 0; h < NSL; ++h) so[h] = lane + 64 * h <= a ? sp[lane + 64 * h] : 0;
+        }
+    };
+    if (k < k1) fetch(k, code, 0, v, sl);
+    while (k < k1) {
+        const int a = (int)(code & 1023), len = 9 * a + 6;
+        // the group after this one
+        int64_t kn = k, cn = code;
+        int xn = x0 + 64 * RG;
+        if (xn >= len) {
+            ++kn;
+            xn = 0;
+            cn = next;   // loaded an incidence ahead of its run
+            next = kn + 1 < k1 ? irow[kn + 1] : 0;
+        }
+        double w[RG];
+        uint16_t sn[NSL];
+#pragma unroll
+        for (int h = 0; h < NSL; ++h) sn[h] = sl[h];
+        if (kn < k1) fetch(kn, cn, xn, w, sn);
+#pragma unroll
+        for (int u = 0; u < RG; ++u) {
+            // uniform: the run's last group may be short (at p = 4 the branches cost more than they save)
+            if (NSL == 1 && x0 + 64 * u >= len) break;
+            const int x = x0 + lane + 64 * u;
+            const int b = (x * 7282) >> 16;   // x / 9 for x < 7282
+            int slot = __shfl((int)sl[0], b & 63, 64);
+            if (NSL > 1) {
+                const int s1 = __shfl((int)sl[NSL - 1], b & 63, 64);
+                slot = b < 64 ? slot : s1;
+            }
+            double *p = acc + 9 * slot;
+            const int m = x - 9 * b;
+            if (b < a) {
+                p[m] += v[u];
+            } else if (x < len) {   // diagonal block: (0,0) (0,1) (1,1) (0,2) (1,2) (2,2), side + side^T
+                const int kk = (0x210100 >> (4 * m)) & 15, ll = (0x222110 >> (4 * m)) & 15;
+                p[3 * kk + ll] += kk == ll ? 2.0 * v[u] : v[u];
+                if (kk != ll) p[3 * ll + kk] += v[u];
+            }
+        }
+#pragma unroll
+        for (int u = 0; u < RG; ++u) v[u] = w[u];
+#pragma unroll
+        for (int h = 0; h < NSL; ++h) sl[h] = sn[h];
+        k = kn;
+        code = cn;
+        x0 = xn;
+    }
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    // row I: 3 nu consecutive values for each dof
+    for (int kk = 0; kk < 3; ++kk) {
+        double *o = vals + 9 * b0 + 3LL * kk * nb + 3 * jd;
+        for (int y = lane; y < 3 * nu; y += 64) {
+            const int j = y / 3;
+            o[y] = acc[9 * j + 3 * kk + (y - 3 * j)];
+        }
+    }
+    // the transposes, in the rows of the blocks' columns
+    for (int j = 1 + lane; j < nu; j += 64) {
+        const int32_t J = bcol[b0 + jd + j];
+        const int64_t m0 = bptr[J];
+        const int mb = (int)(bptr[J + 1] - m0);
+        double *o = vals + 9 * m0 + 3 * (int)mirror[b0 + jd + j];
+#pragma unroll
+        for (int kk = 0; kk < 3; ++kk)
+#pragma unroll
+            for (int l = 0; l < 3; ++l) o[3LL * kk * mb + l] = acc[9 * j + 3 * l + kk];
+    }
+}
+
+// Per CP row: the element rows and slots of its incidences; flags[0]: most blocks J >= I of a row,
+// flags[1]: set when some element has a CP J_b < I_a with b < a (numbered otherwise).
+__global__ void __launch_bounds__(64) slot_kernel(int32_t nb_cp, const int64_t *inc_ptr, const int64_t *inc, PatchIen pi,
+                                                  const int64_t *bptr, const int32_t *bcol, const int32_t *bdiag,
+                                                  int32_t sstride, int64_t *irow, uint16_t *slots, int32_t *flags) {
+    const int row = blockIdx.x, lane = threadIdx.x;
+    if (row >= nb_cp) return;
+    const int64_t b0 = bptr[row];
+    const int nb = (int)(bptr[row + 1] - b0), jd = bdiag[row];
+    if (lane == 0) atomicMax(&flags[0], nb - jd);
+    bool other = false;
+    for (int64_t k = inc_ptr[row]; k < inc_ptr[row + 1]; ++k) {
+        const int64_t en = inc[k];
+        const int patch = (int)(en >> 58), ea = (int)((en >> 10) & ((1LL << 48) - 1)), a = (int)(en & 1023);
+        const int nn = pi.nn[patch];
+        const int32_t *ie = pi.ien[patch] + (int64_t)nn * pi.elems[patch][ea];
+        if (lane == 0) irow[k] = ((pi.offs[patch][ea] + (9LL * a * a + 3LL * a) / 2) << 10) | a;
+        for (int b = lane; b <= a; b += 64) {
+            const int32_t J = ie[b] - 1;
+            if (J < row || (b < a && J == row)) {
+                other = true;
+                continue;
+            }
+            int lo = jd, hi = nb - 1;
+            while (lo < hi) {
+                const int mid = (lo + hi) >> 1;
+                if (bcol[b0 + mid] < J) lo = mid + 1; else hi = mid;
+            }
+            slots[k * sstride + b] = (uint16_t)(lo - jd);
+        }
+    }
+    if (other) atomicOr(&flags[1], 1);
 }
 
 // ---- SpMV by nodal 3x3 blocks: one wave per CP row ---------------------------------------
@@ -547,20 +765,56 @@ int32_t yeti_csr_create(const yeti_asm *h, void *stream, yeti_csr **out) {
         return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc bcol"));
     hipLaunchKernelGGL(row_pattern_kernel<true>, dim3((v.nb_cp + 3) / 4), dim3(256), 0, st, v.nb_cp, inc_ptr.p,
                        inc.p, pi, nullptr, c->bptr.p, c->bcol.p, oflow.p);
-    // contributions
-    if (bcount.alloc(std::max<int64_t>(c->nblocks, 1)) != hipSuccess ||
-        c->cptr.alloc(c->nblocks + 1) != hipSuccess)
-        return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc contributions"));
-    hipLaunchKernelGGL(contrib_kernel<false>, dim3(v.nb_cp), dim3(64), 0, st, v.nb_cp, inc_ptr.p, inc.p, pi,
-                       c->bptr.p, c->bcol.p, bcount.p, nullptr, nullptr);
-    if ((rc = exclusive_scan<int32_t>(bcount.p, c->nblocks, c->cptr.p, st))) return fail(rc);
-    int64_t ncontrib = 0;
-    if (hipMemcpy(&ncontrib, c->cptr.p + c->nblocks, 8, hipMemcpyDeviceToHost) != hipSuccess)
-        return fail(set_error(YETI_ERR_DEVICE, "CSR: copy failed"));
-    if (c->contrib.alloc(std::max<int64_t>(ncontrib, 1)) != hipSuccess)
-        return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc contrib list (%lld entries)", (long long)ncontrib));
-    hipLaunchKernelGGL(contrib_kernel<true>, dim3(v.nb_cp), dim3(64), 0, st, v.nb_cp, inc_ptr.p, inc.p, pi,
-                       c->bptr.p, c->bcol.p, nullptr, c->cptr.p, c->contrib.p);
+    if (c->bdiag.alloc(std::max<int64_t>(v.nb_cp, 1)) != hipSuccess ||
+        c->mirror.alloc(std::max<int64_t>(c->nblocks, 1)) != hipSuccess)
+        return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc mirror"));
+    hipLaunchKernelGGL(mirror_kernel, dim3((v.nb_cp + 3) / 4), dim3(256), 0, st, v.nb_cp, c->bptr.p, c->bcol.p, c->bdiag.p,
+                       c->mirror.p);
+    // element rows, when every element is numbered against its CPs and rows are long enough
+    // (csr_values_kernel packs short rows: at p = 1 a run is 36 entries on average)
+    int32_t nn_max = 1;
+    for (int p = 0; p < v.npatch; ++p)
+        if (v.n_active[p] > 0) nn_max = std::max(nn_max, v.nnode[p]);
+    const int64_t mean = (c->nblocks / std::max(v.nb_cp, 1) + 1) / 2;
+    if (mean > 32 && nn_max <= 128) {
+        DevBuf<int32_t> flags;
+        int32_t fl[2] = {0, 1};
+        c->sstride = nn_max;
+        if (flags.alloc(2) != hipSuccess || hipMemsetAsync(flags.p, 0, 8, st) != hipSuccess ||
+            c->irow.alloc(std::max<int64_t>(ninc, 1)) != hipSuccess ||
+            c->slots.alloc((size_t)std::max<int64_t>(ninc, 1) * nn_max) != hipSuccess)
+            return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc element rows"));
+        hipLaunchKernelGGL(slot_kernel, dim3(v.nb_cp), dim3(64), 0, st, v.nb_cp, inc_ptr.p, inc.p, pi, c->bptr.p, c->bcol.p,
+                           c->bdiag.p, c->sstride, c->irow.p, c->slots.p, flags.p);
+        if (hipMemcpyAsync(fl, flags.p, 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
+            hipStreamSynchronize(st) != hipSuccess)
+            return fail(set_error(YETI_ERR_DEVICE, "CSR: copy failed"));
+        if (fl[1] == 0 && (size_t)fl[0] * 72 * ROW_WAVES <= 64 * 1024) {
+            c->upper = fl[0];
+            if (c->iptr.alloc(v.nb_cp + 1) != hipSuccess ||
+                hipMemcpyAsync(c->iptr.p, inc_ptr.p, 8 * (size_t)(v.nb_cp + 1), hipMemcpyDeviceToDevice, st) != hipSuccess)
+                return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc element rows"));
+        } else {
+            c->irow.release();
+            c->slots.release();
+        }
+    }
+    // contributions per block
+    if (c->upper == 0) {
+        if (bcount.alloc(std::max<int64_t>(c->nblocks, 1)) != hipSuccess ||
+            c->cptr.alloc(c->nblocks + 1) != hipSuccess)
+            return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc contributions"));
+        hipLaunchKernelGGL(contrib_kernel<false>, dim3(v.nb_cp), dim3(64), 0, st, v.nb_cp, inc_ptr.p, inc.p, pi,
+                           c->bptr.p, c->bcol.p, bcount.p, nullptr, nullptr);
+        if ((rc = exclusive_scan<int32_t>(bcount.p, c->nblocks, c->cptr.p, st))) return fail(rc);
+        int64_t ncontrib = 0;
+        if (hipMemcpy(&ncontrib, c->cptr.p + c->nblocks, 8, hipMemcpyDeviceToHost) != hipSuccess)
+            return fail(set_error(YETI_ERR_DEVICE, "CSR: copy failed"));
+        if (c->contrib.alloc(std::max<int64_t>(ncontrib, 1)) != hipSuccess)
+            return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc contrib list (%lld entries)", (long long)ncontrib));
+        hipLaunchKernelGGL(contrib_kernel<true>, dim3(v.nb_cp), dim3(64), 0, st, v.nb_cp, inc_ptr.p, inc.p, pi,
+                           c->bptr.p, c->bcol.p, nullptr, c->cptr.p, c->contrib.p);
+    }
     // scalar pattern
     if (c->rowptr.alloc(3 * (int64_t)v.nb_cp + 1) != hipSuccess ||
         c->colind.alloc(std::max<int64_t>(9 * c->nblocks, 1)) != hipSuccess)
@@ -581,8 +835,29 @@ const int32_t *yeti_csr_colind(const yeti_csr *c) { return c ? c->colind.p : nul
 int32_t yeti_csr_values(const yeti_csr *c, const double *Kdata_dev, double *vals_dev, void *stream) {
     if (!c || !Kdata_dev || !vals_dev) return set_error(YETI_ERR_INVALID_ARGUMENT, "null argument");
     if (c->nblocks == 0) return 0;
-    hipLaunchKernelGGL(csr_values_kernel, dim3((unsigned)((c->nblocks + 255) / 256)), dim3(256), 0,
-                       (hipStream_t)stream, c->nb_cp, c->bptr.p, c->cptr.p, c->contrib.p, Kdata_dev, vals_dev);
+    if (c->upper > 0) {
+        auto rows = [&](auto kern) {
+            hipLaunchKernelGGL(kern, dim3(xcd_grid(((int64_t)c->nb_cp + ROW_WAVES - 1) / ROW_WAVES)), dim3(64 * ROW_WAVES),
+                               (size_t)c->upper * 72 * ROW_WAVES, (hipStream_t)stream, c->nb_cp, c->upper, c->sstride,
+                               c->bptr.p, c->bcol.p, c->bdiag.p, c->mirror.p, c->iptr.p, c->irow.p, c->slots.p, Kdata_dev,
+                               vals_dev);
+        };
+        if (c->sstride <= 64) rows(row_values_kernel<1>);
+        else rows(row_values_kernel<2>);
+        YETI_HIP(hipGetLastError());
+        return 0;
+    }
+    // lanes per row: the mean number of its blocks J >= I (p = 1: 14 of a row's 27), so that short rows
+    // share a wave
+    const int64_t mean = (c->nblocks / std::max(c->nb_cp, 1) + 1) / 2;
+    auto go = [&](auto kern, int rows) {
+        hipLaunchKernelGGL(kern, dim3(xcd_grid(((int64_t)c->nb_cp + rows - 1) / rows)), dim3(256), 0, (hipStream_t)stream,
+                           c->nb_cp, c->bptr.p, c->bcol.p, c->bdiag.p, c->mirror.p, c->cptr.p, c->contrib.p, Kdata_dev,
+                           vals_dev);
+    };
+    if (mean <= 16) go(csr_values_kernel<16>, 16);
+    else if (mean <= 32) go(csr_values_kernel<32>, 8);
+    else go(csr_values_kernel<64>, 4);
     YETI_HIP(hipGetLastError());
     return 0;
 }
