@@ -177,3 +177,30 @@ def test_load_point_chunks_match_oracle(gpu, p, ng):
     F = sys_linmat_lindef_static(**a)[3]
     F0 = O.oracle_sys_linmat((), kwargs=a)[3]
     assert np.abs(F - F0).max() <= 1e-12 * np.abs(F0).max()
+
+
+@pytest.mark.parametrize("nel", [(1, 1, 1), (3, 2, 1), (13, 11, 16)])
+def test_p3_kernel_runs_and_offsets(gpu, nel):
+    """The p = 3 kernel with one element, with fewer elements than the 8 runs they are dealt in, and
+    with runs of unequal length and several elements per workgroup; inactive elements; outputs at
+    an even and an odd address: indices bit-exact, values within 1e-12 of their maximum of the
+    oracle, values only the same bits."""
+    import torch
+    from yeti_amd.assembly import Assembler
+    print("[case] p=3 kernel", nel, flush=True)
+    a = dict(make_box_patch(nel=nel, p=3, seed=12).args)
+    if a["nb_elem"] > 2:
+        a["activeElement"] = a["activeElement"].copy()
+        a["activeElement"][[1, -1]] = 0
+    Ko, ro, co, _ = O.oracle_sys_linmat((), kwargs=a)
+    asm = Assembler(a)
+    n = asm.nb_data
+    for off in (0, 1):
+        K = torch.zeros(n + 2, dtype=torch.float64, device="cuda")[off:]
+        r, c = (torch.zeros(n + 4, dtype=torch.int32, device="cuda")[k + off:] for k in (0, 1))
+        asm.run_matrix(K, r, c)
+        assert np.array_equal(r[:n].cpu().numpy(), ro[:n]) and np.array_equal(c[:n].cpu().numpy(), co[:n])
+        assert np.abs(K[:n].cpu().numpy() - Ko[:n]).max() <= 1e-12 * np.abs(Ko).max()
+        V = torch.zeros(n + 1, dtype=torch.float64, device="cuda")
+        asm.run_values(V)
+        assert torch.equal(V[:n], K[:n]) and float(K[n:].abs().max()) == 0.0

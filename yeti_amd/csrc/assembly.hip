@@ -27,6 +27,7 @@
 
 #include "common.hpp"
 #include "elem_general.hpp"
+#include "elem_p3.hpp"
 
 namespace yeti {
 
@@ -818,7 +819,7 @@ static int gauss_per_dir(int nbint) {
     return n;
 }
 
-// elem_stiffness_kernel is built for p = 3 and 4 with p + 1 Gauss points per direction
+// elem_p3_kernel and elem_stiffness_kernel (p = 4) take p + 1 Gauss points per direction
 static bool fixed_kernel_available(int p0, int p1, int p2, int ng) {
     return p0 == p1 && p1 == p2 && (p0 == 3 || p0 == 4) && ng == p0 + 1;
 }
@@ -826,7 +827,7 @@ static bool fixed_kernel_available(int p0, int p1, int p2, int ng) {
 // every other case goes to elem_general.hip: up to 64 nodes, degrees up to 4, up to 9 points. (p = 1
 // and 2 as well: one wave per 16-node tile pair and several workgroups per CU against one persistent
 // workgroup, 64^3 p = 1 1.39 -> 1.19 ms, p = 2 6.23 -> 5.07 ms with indices; at 32^3 p = 3 it takes 5.23
-// against 3.08 ms.)
+// ms, elem_p3_kernel 1.95.)
 static bool kernel_available(int p0, int p1, int p2, int ng) {
     if (fixed_kernel_available(p0, p1, p2, ng)) return true;
     return p0 >= 1 && p1 >= 1 && p2 >= 1 && p0 <= 4 && p1 <= 4 && p2 <= 4 && (p0 + 1) * (p1 + 1) * (p2 + 1) <= 64 &&
@@ -922,20 +923,23 @@ static int launch_elem(yeti_asm *h, PatchDev &pd, const double *coords, double *
         constexpr int GEO_EPB = 4 * geo_epw<C::NQ>();
         hipLaunchKernelGGL((elem_geo_kernel<P, NG>), dim3((unsigned)((pa.n_active + GEO_EPB - 1) / GEO_EPB)), dim3(256), 0,
                            st, pa, pd.geo.p);
-        // persistent workgroups: one per CU (the kernel's LDS and registers allow one)
-        const int grid = std::min(pa.n_active, cus);
         hipEvent_t ea = nullptr, eb = nullptr;
         if (h->timing) {
             int rc = timing_events(h, h->ev_used++, &ea, &eb);
             if (rc) return rc;
             YETI_HIP(hipEventRecord(ea, st));
         }
-        if (Kr || C::VALUES_VIA_IDX)
+        if constexpr (P == 3) {
+            int rc = launch_elem_p3(pd.geo.p, pa.offs, pa.n_active, pa.lam, pa.mu, cus, Kd, Kr, Kc, st);
+            if (rc) return rc;
+        } else {
+            // persistent workgroups: one per CU (the kernel's LDS and registers allow one). Values-only
+            // runs take this instantiation too, with null index pointers (ElemCfg::VALUES_VIA_IDX)
+            static_assert(C::VALUES_VIA_IDX, "one instantiation");
+            const int grid = std::min(pa.n_active, cus);
             hipLaunchKernelGGL((elem_stiffness_kernel<P, NG, true>), dim3(grid), dim3(C::NTH), 0, st, pa,
                                (const double *)pd.geo.p, Kd, Kr, Kc);
-        else
-            hipLaunchKernelGGL((elem_stiffness_kernel<P, NG, false>), dim3(grid), dim3(C::NTH), 0, st, pa,
-                               (const double *)pd.geo.p, Kd, Kr, Kc);
+        }
         YETI_HIP(hipGetLastError());
         if (h->timing) YETI_HIP(hipEventRecord(eb, st));
     }

@@ -17,11 +17,9 @@ namespace yeti {
 constexpr int XCDS = 8;
 
 // grid of a one-element-per-workgroup kernel and the element of workgroup b (>= n: none)
-inline unsigned xcd_grid(int64_t n) { return (unsigned)((n + XCDS - 1) / XCDS * XCDS); }
-__device__ __forceinline__ int64_t xcd_element(int64_t b, int64_t n) {
-    const int64_t per = (n + XCDS - 1) / XCDS;
-    return b % XCDS * per + b / XCDS;
-}
+__host__ __device__ inline int64_t xcd_per(int64_t n) { return (n + XCDS - 1) / XCDS; }
+inline unsigned xcd_grid(int64_t n) { return (unsigned)(xcd_per(n) * XCDS); }
+__device__ __forceinline__ int64_t xcd_element(int64_t b, int64_t n) { return b % XCDS * xcd_per(n) + b / XCDS; }
 
 // dst[x] = get(x), x < n, by threads t of NTH
 template <int NTH, typename T, typename F>
