@@ -181,11 +181,12 @@ def test_gpu_general_degrees_postprocessing_match_oracle(name):
 
 @pytest.mark.gpu
 @pytest.mark.parametrize("deg,nel,ng", [((1, 1, 1), (3, 3, 1), 2), ((2, 2, 2), (5, 1, 2), 3), ((4, 2, 1), (2, 2, 2), 5),
-                                        ((3, 3, 2), (2, 1, 2), 4), ((3, 4, 2), (1, 2, 1), 5), ((3, 3, 3), (1, 1, 2), 9)])
+                                        ((3, 3, 2), (2, 1, 2), 4), ((3, 4, 2), (1, 2, 1), 5), ((3, 3, 3), (1, 1, 2), 9),
+                                        ((4, 4, 4), (3, 2, 2), 5)])
 def test_gpu_general_kernel_tiles_and_offsets(deg, nel, ng):
-    """elem_general at 8 to 64 nodes (one to four node tiles, full and partly filled; above 32
-    nodes the entries leave in several rounds), 8 to 729 points (whole and partial chunks),
-    elements whose COO range starts at odd entries and at every inactive-element offset, and
+    """elem_general at 8 to 64 nodes and at 125 (one to four or eight node tiles, full and partly
+    filled; above 32 nodes the entries leave in several rounds), 8 to 729 points (whole and partial
+    chunks), elements whose COO range starts at odd entries and at every inactive-element offset, and
     outputs at an odd address: stiffness and mass against the oracle, indices bit-exact, values
     within 1e-12 of their maximum."""
     import torch

@@ -136,7 +136,7 @@ __host__ __device__ inline void bspline_ders(int i, double u, const double *__re
     }
 }
 
-#include "elem_kernel.hpp"
+#include "elem_geo.hpp"
 #include "shape_grad.hpp"
 
 // ------------------------------------------------------------------------------------------
@@ -819,7 +819,7 @@ static int gauss_per_dir(int nbint) {
     return n;
 }
 
-// elem_p3_kernel and elem_stiffness_kernel (p = 4) take p + 1 Gauss points per direction
+// elem_p3_kernel and elem_general_kernel<8, 0> (p = 4) take p + 1 Gauss points per direction
 static bool fixed_kernel_available(int p0, int p1, int p2, int ng) {
     return p0 == p1 && p1 == p2 && (p0 == 3 || p0 == 4) && ng == p0 + 1;
 }
@@ -896,6 +896,28 @@ static int timing_events(yeti_asm *h, int k, hipEvent_t *a, hipEvent_t *b) {
     return 0;
 }
 
+static GenArgs general_args(yeti_asm *h, PatchDev &pd) {
+    GenArgs ga{};
+    ga.coords = h->coords.p;
+    ga.ien = pd.ien.p;
+    ga.weight = pd.weight.p;
+    ga.nijk = pd.nijk.p;
+    for (int d = 0; d < 3; ++d) {
+        ga.tab[d] = pd.tab[d].p;
+        ga.n[d] = pd.p[d] + 1;
+    }
+    ga.elems = pd.elems.p;
+    ga.offs = pd.offs.p;
+    ga.n_active = pd.n_active;
+    ga.tab_n = pd.tab_n;
+    ga.ng = pd.ng;
+    ga.lam = pd.lam;
+    ga.mu = pd.mu;
+    ga.rho = pd.rho;
+    gauss_legendre(pd.ng, ga.g.x, ga.g.w);
+    return ga;
+}
+
 template <int P, int NG>
 static int launch_elem(yeti_asm *h, PatchDev &pd, const double *coords, double *Kd, int32_t *Kr, int32_t *Kc,
                        hipStream_t st) {
@@ -920,7 +942,7 @@ static int launch_elem(yeti_asm *h, PatchDev &pd, const double *coords, double *
         pa.elems = pd.elems.p + e0;
         pa.offs = pd.offs.p + e0;
         pa.n_active = std::min(batch, pd.n_active - e0);
-        constexpr int GEO_EPB = 4 * geo_epw<C::NQ>();
+        constexpr int GEO_EPB = 4;   // elements per workgroup, one wave each
         hipLaunchKernelGGL((elem_geo_kernel<P, NG>), dim3((unsigned)((pa.n_active + GEO_EPB - 1) / GEO_EPB)), dim3(256), 0,
                            st, pa, pd.geo.p);
         hipEvent_t ea = nullptr, eb = nullptr;
@@ -933,14 +955,15 @@ static int launch_elem(yeti_asm *h, PatchDev &pd, const double *coords, double *
             int rc = launch_elem_p3(pd.geo.p, pa.offs, pa.n_active, pa.lam, pa.mu, cus, Kd, Kr, Kc, st);
             if (rc) return rc;
         } else {
-            // persistent workgroups: one per CU (the kernel's LDS and registers allow one). Values-only
-            // runs take this instantiation too, with null index pointers (ElemCfg::VALUES_VIA_IDX)
-            static_assert(C::VALUES_VIA_IDX, "one instantiation");
-            const int grid = std::min(pa.n_active, cus);
-            hipLaunchKernelGGL((elem_stiffness_kernel<P, NG, true>), dim3(grid), dim3(C::NTH), 0, st, pa,
-                               (const double *)pd.geo.p, Kd, Kr, Kc);
+            GenArgs ga = general_args(h, pd);
+            ga.elems = pa.elems;
+            ga.offs = pa.offs;
+            ga.n_active = pa.n_active;
+            ga.geo = pd.geo.p;
+            ga.geo_rec = C::REC;
+            int rc = launch_elem_general(ga, false, Kd, Kr, Kc, st);
+            if (rc) return rc;
         }
-        YETI_HIP(hipGetLastError());
         if (h->timing) YETI_HIP(hipEventRecord(eb, st));
     }
     return 0;
@@ -949,24 +972,7 @@ static int launch_elem(yeti_asm *h, PatchDev &pd, const double *coords, double *
 // Degree triples and Gauss orders the fixed-degree kernels are not built for (elem_general.hip).
 static int launch_generic(yeti_asm *h, PatchDev &pd, double *Kd, int32_t *Kr, int32_t *Kc, hipStream_t st,
                           bool mass = false) {
-    GenArgs ga{};
-    ga.coords = h->coords.p;
-    ga.ien = pd.ien.p;
-    ga.weight = pd.weight.p;
-    ga.nijk = pd.nijk.p;
-    for (int d = 0; d < 3; ++d) {
-        ga.tab[d] = pd.tab[d].p;
-        ga.n[d] = pd.p[d] + 1;
-    }
-    ga.elems = pd.elems.p;
-    ga.offs = pd.offs.p;
-    ga.n_active = pd.n_active;
-    ga.tab_n = pd.tab_n;
-    ga.ng = pd.ng;
-    ga.lam = pd.lam;
-    ga.mu = pd.mu;
-    ga.rho = pd.rho;
-    gauss_legendre(pd.ng, ga.g.x, ga.g.w);
+    const GenArgs ga = general_args(h, pd);
     hipEvent_t ea = nullptr, eb = nullptr;
     if (h->timing && !mass) {
         int rc = timing_events(h, h->ev_used++, &ea, &eb);

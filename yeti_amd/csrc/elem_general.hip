@@ -1,5 +1,5 @@
 // elem_general.hip -- element stiffness and mass matrices for run-time degrees and Gauss orders,
-// up to 64 nodes, on the FP64 matrix cores.
+// up to 64 nodes, and stiffness at p = 4, on the FP64 matrix cores.
 //
 // Stiffness: K_ab[k][l] = lam S^kl_ab + mu S^lk_ab + mu delta_kl tr S_ab with
 // S^kl_ab = sum_q G_k[a][q] G_l[b][q], G_c[a][q] = sqrt(w_q |det J_q|) dR_a/dx_c (UELMAT.f90:22-225 with
@@ -28,18 +28,33 @@ typedef double f64x2 __attribute__((ext_vector_type(2)));
 // 5.07 ms without the stores, whose floor is 2.1 ms; the mass at 61x53x47 p = 2 takes 1.0 of 2.12 ms.
 // Against vector sums of every node pair from LDS and block-wise stores: 45x14x11 degrees (2,3,1)
 // 1018 -> 216 us; mass 61x53x47 p = 2 2.94 -> 2.12 ms, 64^3 p = 1 1.91 -> 0.69 ms.
+// NT = 8 (125 nodes): 36 pairs of nine tiles are more accumulators than a CU has registers for, hence
+// four workgroups per element. Each builds G again and no two fit a CU (stage of 120 KB); at 23x18x13
+// the matrix instructions of the busiest SIMD take 1.6 of 3.76 ms (at 2.4 GHz). Against one persistent
+// workgroup of 12 waves, 4 of them building G, with spilled accumulators: values 5.18 -> 3.76 ms, with
+// indices 6.05 -> 4.27 ms, 4x4x4 296 -> 95 us. One half for G and two barriers per chunk: 3.90 ms.
 template <int NT, int MODE>
 struct Gen {
-    static constexpr int NNP = 16 * NT, WAVES = NT * (NT + 1) / 2;
+    static constexpr int NNP = 16 * NT;
+    // a workgroup takes an element, or at NT = 8 (p = 4) a quarter of it: the tile columns 0-3, 4-5, 6
+    // or 7 (10, 11, 7 and 8 pairs) on 11 waves, its geometry from the record of elem_geo_kernel
+    static constexpr int PASSES = NT == 8 ? 4 : 1;
+    static constexpr int WAVES = NT == 8 ? 11 : NT * (NT + 1) / 2;
     static constexpr int NTH = 64 * WAVES;
     static constexpr int QC = NT <= 2 ? 32 : 16;            // Gauss points per chunk
+    __host__ __device__ static constexpr int column(int pass) {   // first tile column of a pass
+        return NT != 8 ? (pass == 0 ? 0 : NT) : pass == 0 ? 0 : pass == 1 ? 4 : pass == 2 ? 6 : pass == 3 ? 7 : 8;
+    }
     static constexpr int PARTS = NT == 1 ? 2 : NT == 2 ? 4 : 16;   // lanes per point, step 1
     static constexpr int RS = QC + 2;                       // G row (doubles): rows on different banks
     static constexpr int NG_ = MODE == 0 ? 3 : 1;           // arrays per node
     static constexpr int TILES = MODE == 0 ? 9 : 1;
     static constexpr int GDBL = NG_ * NNP * RS;
+    // NT = 8: the chunks alternate between two halves, one barrier each; a half is written again once
+    // every wave has met the barrier after its last read
+    static constexpr int GBUF = NT == 8 ? 2 : 1;
     static constexpr int WPE = MODE == 1 ? 4 : 3;           // waves per SIMD
-    static_assert(PARTS * QC <= NTH, "one pass over the chunk's points");
+    static_assert(NT == 8 || PARTS * QC <= NTH, "one pass over the chunk's points");
 };
 
 constexpr int GEN_NGEO = 12;
@@ -92,7 +107,8 @@ __host__ __device__ constexpr int gen_round_entries(int nn) {
 template <int NT, int MODE>
 __host__ __device__ constexpr int gen_values(int nn) {
     const int v = MODE == 1 ? 1 + nn * (nn + 1) / 2 : gen_round_entries<NT>(nn);
-    return v > Gen<NT, MODE>::GDBL ? v : Gen<NT, MODE>::GDBL;
+    constexpr int g = Gen<NT, MODE>::GBUF * Gen<NT, MODE>::GDBL;
+    return v > g ? v : g;
 }
 
 template <int NT, int MODE, bool IDX>
@@ -103,7 +119,7 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
     // G of a chunk; after the last one the values of a round; for the mass then the round's rows of
     // entry_tab (a load among the stores of the copy would wait for them: one counter covers both)
     extern __shared__ __attribute__((aligned(16))) double sm[];
-    __shared__ __attribute__((aligned(16))) double gq[MODE == 0 ? GEN_NGEO : 2][QC];   // sqrt(dv) dxi_m/dx_c / W (9), dW/dxi_m / W (3); mass: 1/W, dv
+    __shared__ __attribute__((aligned(16))) double gq[MODE == 0 ? GEN_NGEO : 2][NT == 8 ? 2 : QC];   // sqrt(dv) dxi_m/dx_c / W (9), dW/dxi_m / W (3); mass: 1/W, dv
     __shared__ double tb[3][2 * MAX_NG * (GEN_MAXP + 1) + 2];   // per direction: [B | dB][g][i], half span
     __shared__ __attribute__((aligned(16))) double xw[NNP][4];
     __shared__ int32_t dof[3 * NNP];
@@ -115,8 +131,10 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
     // one element per workgroup (a loop over elements would keep the entries' indices in registers
     // from one to the next)
     {
-        const int64_t gi = xcd_element(blockIdx.x, ga.n_active);
-        if (gi >= ga.n_active) return;
+        const int64_t item = xcd_element(blockIdx.x, (int64_t)ga.n_active * C::PASSES);
+        if (item >= (int64_t)ga.n_active * C::PASSES) return;
+        const int64_t gi = item / C::PASSES;
+        const int pass = (int)(item % C::PASSES), J0 = C::column(pass), J1 = C::column(pass + 1);
         const int e = ga.elems[gi];
         for (int a = t; a < NNP; a += NTH) {
             const bool in = a < NN;
@@ -145,14 +163,24 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
         f64x4 acc[TILES];
 #pragma unroll
         for (int s = 0; s < TILES; ++s) acc[s] = f64x4{0.0, 0.0, 0.0, 0.0};
-        // pair of the wave, column by column: wv = J (J + 1) / 2 + I
-        const int J = wv < 1 ? 0 : wv < 3 ? 1 : wv < 6 ? 2 : 3, I = wv - J * (J + 1) / 2;
+        // pair of the wave, column by column: pr = J (J + 1) / 2 + I
+        const int pr = J0 * (J0 + 1) / 2 + wv;
+        const int J = pr < 1 ? 0 : pr < 3 ? 1 : pr < 6 ? 2 : pr < 10 ? 3 : pr < 15 ? 4 : pr < 21 ? 5 : pr < 28 ? 6 : 7;
+        const int I = pr - J * (J + 1) / 2;
+        const bool has = J < J1 && I <= J;   // not a wave beyond the pass's pairs
+        // NT = 8: the thread's point of the next chunk, from the record ([12][points], xi_0 fastest)
+        const double *geo = NT == 8 ? ga.geo + gi * ga.geo_rec : nullptr;
+        double Ap[NT == 8 ? GEN_NGEO : 1];
+        if constexpr (NT == 8) {
+#pragma unroll
+            for (int m = 0; m < GEN_NGEO; ++m) Ap[m] = geo[m * NQ + min(t % QC, NQ - 1)];
+        }
         __syncthreads();
         for (int q0 = 0; q0 < NQ; q0 += QC) {
             const int nq = min(NQ - q0, QC);
             // 1. geometry of the chunk's points (3D rule: i slowest, k fastest, GaussLegendre.f90:175-186):
             // along a node line (j, k) first, then the line's sums with its xi_1, xi_2 functions
-            {
+            if constexpr (NT != 8) {
                 const int qq = t / C::PARTS, part = t % C::PARTS;
                 double s[16];
 #pragma unroll
@@ -227,20 +255,25 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
                     gq[1][qq] = 0.0;
                 }
             }
-            __syncthreads();
+            if (NT != 8) __syncthreads();
+            double *smg = C::GBUF == 2 ? sm + (q0 / QC % 2) * C::GDBL : sm;
             // 2. G of the chunk, zero past the nodes and past the points (up to a multiple of 8)
             {
                 constexpr int PER = NTH / QC;      // threads per point
                 const int qq = t % QC, part = t / QC, nq8 = (nq + 7) & ~7;
                 if (part < PER && qq < nq8) {
                     const bool inq = qq < nq;
-                    const int q = inq ? q0 + qq : q0, g0 = div_by(q, mg2), g1 = div_by(q - g0 * ng * ng, mg),
-                              g2 = q - ng * (ng * g0 + g1);
+                    const int q = inq ? q0 + qq : q0, qs = div_by(q, mg2), g1 = div_by(q - qs * ng * ng, mg),
+                              qf = q - ng * (ng * qs + g1);
+                    const int g0 = NT == 8 ? qf : qs, g2 = NT == 8 ? qs : qf;
                     const double *T0 = &tb[0][g0 * TN], *T1 = &tb[1][g1 * TN], *T2 = &tb[2][g2 * TN];
                     const int dB = ng * TN;
                     double A[GEN_NGEO];
 #pragma unroll
-                    for (int m = 0; m < (MODE == 0 ? GEN_NGEO : 1); ++m) A[m] = inq ? gq[m][qq] : 0.0;
+                    for (int m = 0; m < (MODE == 0 ? GEN_NGEO : 1); ++m) {
+                        if constexpr (NT == 8) A[m] = inq ? Ap[m] : 0.0;
+                        else A[m] = inq ? gq[m][qq] : 0.0;
+                    }
                     for (int l = part; l < NL; l += PER) {
                         const int k = div_by(l, mn1), j = l - n1 * k;
                         const double b1 = T1[j], b2 = T2[k], b12 = b1 * b2, d1 = T1[dB + j] * b2, d2 = b1 * T2[dB + k];
@@ -253,20 +286,25 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
                                 const double t2 = bw * d2 - N * A[11];
 #pragma unroll
                                 for (int c = 0; c < 3; ++c)
-                                    sm[(c * NNP + a) * RS + qq] = t0 * A[c] + t1 * A[3 + c] + t2 * A[6 + c];
+                                    smg[(c * NNP + a) * RS + qq] = t0 * A[c] + t1 * A[3 + c] + t2 * A[6 + c];
                             } else {
-                                sm[a * RS + qq] = N * A[0];
+                                smg[a * RS + qq] = N * A[0];
                             }
                         }
                     }
                     for (int a = NN + part; a < NNP; a += PER)
 #pragma unroll
-                        for (int c = 0; c < C::NG_; ++c) sm[(c * NNP + a) * RS + qq] = 0.0;
+                        for (int c = 0; c < C::NG_; ++c) smg[(c * NNP + a) * RS + qq] = 0.0;
                 }
+            }
+            if constexpr (NT == 8) {
+                const int qn = min(q0 + QC + t % QC, NQ - 1);
+#pragma unroll
+                for (int m = 0; m < GEN_NGEO; ++m) Ap[m] = geo[m * NQ + qn];
             }
             __syncthreads();
             // 3. K step 2v uses point 8v + 2 kg, step 2v + 1 point 8v + 2 kg + 1, in A and B alike
-            const int nv = (nq + 7) / 8;
+            const int nv = has ? (nq + 7) / 8 : 0;
 #pragma unroll 1
             for (int v = 0; v < nv; ++v) {
                 const int qo = 8 * v + 2 * kg;
@@ -274,8 +312,8 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
                     f64x2 a[3], b[3];
 #pragma unroll
                     for (int c = 0; c < 3; ++c) {
-                        a[c] = *reinterpret_cast<const f64x2 *>(&sm[(c * NNP + 16 * I + nl) * RS + qo]);
-                        b[c] = *reinterpret_cast<const f64x2 *>(&sm[(c * NNP + 16 * J + nl) * RS + qo]);
+                        a[c] = *reinterpret_cast<const f64x2 *>(&smg[(c * NNP + 16 * I + nl) * RS + qo]);
+                        b[c] = *reinterpret_cast<const f64x2 *>(&smg[(c * NNP + 16 * J + nl) * RS + qo]);
                     }
 #pragma unroll
                     for (int s = 0; s < 9; ++s)
@@ -285,14 +323,15 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
                         acc[s] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[s / 3].y, b[s % 3].y, acc[s], 0, 0, 0);
                 } else {
                     const f64x2 dv = *reinterpret_cast<const f64x2 *>(&gq[1][qo]);
-                    const f64x2 a = *reinterpret_cast<const f64x2 *>(&sm[(16 * I + nl) * RS + qo]) * dv;
-                    const f64x2 b = *reinterpret_cast<const f64x2 *>(&sm[(16 * J + nl) * RS + qo]);
+                    const f64x2 a = *reinterpret_cast<const f64x2 *>(&smg[(16 * I + nl) * RS + qo]) * dv;
+                    const f64x2 b = *reinterpret_cast<const f64x2 *>(&smg[(16 * J + nl) * RS + qo]);
                     acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.x, b.x, acc[0], 0, 0, 0);
                     acc[0] = __builtin_amdgcn_mfma_f64_16x16x4f64(a.y, b.y, acc[0], 0, 0, 0);
                 }
             }
-            __syncthreads();
+            if (C::GBUF == 1) __syncthreads();
         }
+        if (C::GBUF == 2) __syncthreads();
         const int64_t base = ga.offs[gi];
         double *Ke = Kd + base;
         int32_t *Re = IDX ? Kr + base : nullptr, *Ce = IDX ? Kc + base : nullptr;
@@ -308,7 +347,7 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
             }
         }
 #pragma unroll 1
-        for (int rd = 0; rd < ROUNDS; ++rd) {
+        for (int rd = NT == 8 ? J0 : 0; rd < (NT == 8 ? J1 : ROUNDS); ++rd) {
             const int x0 = ROUNDS == 1 ? 0 : gen_coo_start(16 * rd);
             const int x1 = ROUNDS == 1 ? gen_coo_start(NN) : gen_coo_start(min(16 * rd + 16, NN));
             if (ROUNDS > 1 && MODE == 1) load_tab(x0, x1);
@@ -347,12 +386,13 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
                 // columns are loaded now, before the first store
                 typedef uint16_t u16x4 __attribute__((ext_vector_type(4), aligned(2)));
                 typedef int32_t i32x4 __attribute__((ext_vector_type(4), aligned(4)));
-                constexpr int U = IDX ? (gen_round_entries<NT>(NNP) + 4 * NTH - 1) / (4 * NTH) : 1;
+                constexpr bool TAB = IDX && NT != 8;
+                constexpr int U = TAB ? (gen_round_entries<NT>(NNP) + 4 * NTH - 1) / (4 * NTH) : 1;
                 const int n = x1 - x0;
                 u16x4 rc[U];
                 int head = 0, end = 0, xs = -1;   // xs: a single entry before or after the 16-byte ones
                 unsigned rs = 0;
-                if (IDX) {
+                if (TAB) {
                     head = min(n, (int)((0 - reinterpret_cast<uintptr_t>(Re + x0)) / 4 % 32));
                     end = head + (n - head) / 4 * 4;
                     xs = t < head ? t : t - head < n - end ? end + t - head : -1;
@@ -365,7 +405,20 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
                     }
                 }
                 __syncthreads();
-                if (IDX) {
+                if (IDX && NT == 8) {
+                    // 9-bit dofs, which entry_tab does not hold: row by row
+                    for (int b = 16 * rd + wv; b < min(16 * rd + 16, NN); b += C::WAVES) {
+                        int32_t *Rb = Re + gen_coo_start(b), *Cb = Ce + gen_coo_start(b);
+                        for (int y = lane; y < 9 * b + 6; y += 64) {
+                            const int a = y < 9 * b ? y / 9 : b, m = y - 9 * a;
+                            const int kk = a < b ? m % 3 : (0x210100 >> (4 * m)) & 15;
+                            const int ll = a < b ? m / 3 : (0x222110 >> (4 * m)) & 15;
+                            Rb[y] = dof[3 * a + kk];
+                            Cb[y] = dof[3 * b + ll];
+                        }
+                    }
+                }
+                if (TAB) {
                     if (xs >= 0) {
                         Re[x0 + xs] = dof[rs & 255];
                         Ce[x0 + xs] = dof[rs >> 8];
@@ -397,7 +450,7 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
                     store_run<NTH>(Ce + x0, x1 - x0, t, [&](int x) { return dof[et[x] >> 8]; });
                 }
             }
-            if (rd + 1 < ROUNDS) __syncthreads();
+            if (rd + 1 < (NT == 8 ? J1 : ROUNDS)) __syncthreads();
         }
     }
 }
@@ -425,6 +478,15 @@ static void launch_nt(const GenArgs &ga, bool mass, double *Kd, int32_t *Kr, int
 
 int launch_elem_general(const GenArgs &ga, bool mass, double *Kd, int32_t *Kr, int32_t *Kc, hipStream_t st) {
     const int nn = ga.n[0] * ga.n[1] * ga.n[2];
+    if (ga.geo && nn == 125 && ga.tab_n == 5 && ga.ng == 5 && !mass) {
+        if (ga.n_active <= 0) return 0;
+        const size_t lds = gen_smem_bytes<8, 0>(nn);
+        const dim3 grid(xcd_grid((int64_t)ga.n_active * Gen<8, 0>::PASSES)), block(Gen<8, 0>::NTH);
+        if (Kr) hipLaunchKernelGGL((elem_general_kernel<8, 0, true>), grid, block, lds, st, ga, Kd, Kr, Kc);
+        else hipLaunchKernelGGL((elem_general_kernel<8, 0, false>), grid, block, lds, st, ga, Kd, Kr, Kc);
+        YETI_HIP(hipGetLastError());
+        return 0;
+    }
     if (nn < 1 || nn > GEN_MAXN || ga.tab_n < 1 || ga.tab_n > GEN_MAXP + 1 || ga.ng < 1 || ga.ng > MAX_NG)
         return set_error(YETI_ERR_UNSUPPORTED_DEGREE, "general element kernel: %d nodes, %d points", nn, ga.ng);
     if (ga.n_active <= 0) return 0;

@@ -20,10 +20,13 @@ struct GenArgs {
     int32_t tab_n, ng;         // functions per table row, Gauss points per direction
     double lam, mu, rho;
     GaussRule g;
+    const double *geo = nullptr;   // p = 4: geometry records of the elements (elem_geo_kernel), geo_rec apart
+    int64_t geo_rec = 0;
 };
 
 // COO values (and rows / columns, when Kr is given) of the active elements: stiffness, or with
-// `mass` the consistent mass matrix. At most GEN_MAXN nodes and MAX_NG points per direction.
+// `mass` the consistent mass matrix. At most GEN_MAXN nodes and MAX_NG points per direction, or 125
+// nodes and 5 points with geometry records (stiffness).
 int launch_elem_general(const GenArgs &ga, bool mass, double *Kd, int32_t *Kr, int32_t *Kc, hipStream_t st);
 
 }  // namespace yeti
