@@ -696,10 +696,16 @@ def main():
     del u, gs, vol, gvol
     torch.cuda.empty_cache()
 
+    def elem_kernel_name(p, idx):
+        if p == 3:
+            return "elem_p3_kernel<%s>" % str(idx).lower()
+        return "elem_general_kernel<%d,0,%s>" % (((p + 1) ** 3 + 15) // 16, str(idx).lower())
+
     def grad_work(ms, nf):
         """Algorithmic work of one gradient call with nf fields (modes) against the HBM and FP64
         peaks. Per element: IEN, weights, coordinates, spans and the fields' nodal values read,
-        per-node partials and the mass written, then gathered per CP; flops: R and dR/dx per
+        per-node partials and the mass written, then gathered per CP; flops of the direct sums (the
+        kernel contracts direction by direction and does fewer): R and dR/dx per
         (point, node) (~26), u and du/dx per (point, field) (24 per node), the tensor contraction
         per (point, node, field) (18)."""
         n = (p + 1) ** 3
@@ -709,7 +715,7 @@ def main():
         s = ms * 1e-3
         return {"algorithmic_bytes": byts, "achieved_gbs": byts / s / 1e9, "hbm_frac": byts / s / 1e9 / HBM_PEAK_GBS,
                 "flops": flops, "achieved_tflops": flops / s / 1e12, "fp64_frac": flops / s / 1e12 / 78.6,
-                "bound": "latency (one workgroup per element, 5 barriers per Gauss-point chunk)"}
+                "bound": "latency (one wave per element, LDS round trips between the directions)"}
 
     cpu = None
     if not args.no_cpu_baseline:
@@ -741,12 +747,12 @@ def main():
         "roofline": {
             "bound": "hbm", "achieved": achieved, "peak": HBM_PEAK_GBS, "unit": "GB/s",
             "frac": achieved / HBM_PEAK_GBS, "traffic": traffic,
-            "kernel": "elem_stiffness_kernel<%d,%d,true>" % (p, p + 1),
+            "kernel": elem_kernel_name(p, True),
             "kernel_ms": kern_ms, "launches_per_step": nlaunch, "elements_per_launch": elems_per_launch,
             "algorithmic_bytes_per_launch": bytes_launch,
         },
         "mfma_values_only": {
-            "kernel": "elem_stiffness_kernel<%d,%d,false>" % (p, p + 1), "kernel_ms": val_ms,
+            "kernel": elem_kernel_name(p, False), "kernel_ms": val_ms,
             "achieved": tflops, "peak": FP64_PEAK_TFS, "unit": "TFLOP/s",
             "frac": tflops / FP64_PEAK_TFS, "flops_per_launch": elems_per_launch * flops_elem,
         },
