@@ -9,16 +9,10 @@
 //   stiffmatrix_byCP, material_lib   main/stiffmatrix.F90:130-225, main/material_lib.f90:28-98
 //   shapPress                        main/shapPress.f:18-265
 //
-// Element kernel (one workgroup per element):
-//   1. stage the element's CP coordinates, weights, connectivity and the 1D B-spline values /
-//      derivatives at its Gauss abscissae in LDS;
-//   2. per Gauss point, reduce W, dW, sum x N, sum x (x) dN over the nodes -> J^-1, |det J| w;
-//   3. write G_i[q][a] = d R_a / d x_i (q = Gauss point, a = node) to LDS;
-//   4. S^{ij} = G_i^T diag(w|J|) G_j on v_mfma_f64_16x16x4f64: one wave owns whole 16x16 node
-//      tiles (I <= J) and all nine (i, j) component tiles of them, so the isotropic
-//      contraction K_ab[k][l] = lam S^{kl}_ab + mu S^{lk}_ab + mu d_kl tr S_ab is lane-local;
-//   5. emit the element's upper-triangle COO slice in YETI's order (nodj-major, then nodi, then
-//      the 3x3 block column-major; diagonal blocks: the 6 upper entries, diagonal halved).
+// Here: the handle, its tables and the launches; right-hand sides and their gradients; the p = 3 and
+// 4 mass. Element stiffness: elem_p3.hip (p = 3, 4 points per direction) and elem_general.hip (all
+// else); shape gradients: shape_grad.hpp. An element's COO slice is in YETI's order (nodj-major,
+// then nodi, then the 3x3 block column-major; diagonal blocks: the 6 upper entries, diagonal halved).
 #include <algorithm>
 #include <cmath>
 #include <cstring>

@@ -25,7 +25,7 @@
 // = 3. In step A of element e the compute waves fill the first region while the stores of the second
 // one (element e - 1) run; in step B they fill the second one while the first one is stored. A store
 // wave holds the dofs (entry_tab) of all its entries in registers and loads nothing between stores.
-// 64^3 with indices 24.5 -> 15.5 ms per assembly, 40^3 values only 4.89 -> 3.20 ms, against
+// 64^3 with indices 24.3 -> 15.1 ms per assembly, 40^3 values only 4.89 -> 3.20 ms, against
 // warp-specialised products of all node pairs with all points (78 tiles of 16 K steps, chunks of G
 // built beside them). With indices the stores (296 KB per element, 27k cycles at 6.7 TB/s) and the two
 // compute waves of SIMDs 0 and 1 (13k cycles of MFMA) bound it, values only the compute waves.
