@@ -702,16 +702,16 @@ def main():
         return "elem_general_kernel<%d,0,%s>" % (((p + 1) ** 3 + 15) // 16, str(idx).lower())
 
     def grad_work(ms, nf):
-        """Algorithmic work of one gradient call with nf fields (modes) against the HBM and FP64
-        peaks. Per element: IEN, weights, coordinates, spans and the fields' nodal values read,
-        per-node partials and the mass written, then gathered per CP; flops of the direct sums (the
-        kernel contracts direction by direction and does fewer): R and dR/dx per
-        (point, node) (~26), u and du/dx per (point, field) (24 per node), the tensor contraction
-        per (point, node, field) (18)."""
+        """Algorithmic work of one gradient call with nf fields (modes; 0: the volume) against the
+        HBM and FP64 peaks. Per element: IEN, weights, coordinates, spans and the fields' nodal
+        values read, per-node partials and the mass written, then gathered per CP; flops: a
+        quantity with its three derivatives taken to the points, or back to the nodes, direction
+        by direction is 9 (p + 1)^4 multiply-adds: 4 quantities of the map, 3 components per
+        field there and back; about 100 flops per point for the map and 90 per field."""
         n = (p + 1) ** 3
-        nq = (p + 1) ** 3
-        byts = bp.nb_elem * (4 * n + 8 * n + 24 * n + 12 + nf * (24 * n + 24 * n + 8)) + nf * 24 * bp.nb_cp
-        flops = bp.nb_elem * nq * n * (26 + nf * (24 + 18))
+        nb = max(nf, 1)
+        byts = bp.nb_elem * (4 * n + 8 * n + 24 * n + 12 + nf * 24 * n + nb * (24 * n + 8)) + nb * 24 * bp.nb_cp
+        flops = bp.nb_elem * (18 * (p + 1) ** 4 * (4 + 3 * nf + 3 * nb) + n * (100 + 90 * nf))
         s = ms * 1e-3
         return {"algorithmic_bytes": byts, "achieved_gbs": byts / s / 1e9, "hbm_frac": byts / s / 1e9 / HBM_PEAK_GBS,
                 "flops": flops, "achieved_tflops": flops / s / 1e12, "fp64_frac": flops / s / 1e12 / 78.6,
@@ -765,7 +765,7 @@ def main():
                                "work": grad_work(vib_ms, nmode)},
         "strain_energy_gradient": {"ms": seg_ms, "elements_per_s": bp.nb_elem / (seg_ms * 1e-3),
                                    "work": grad_work(seg_ms, 1)},
-        "volume_gradient": {"ms": vol_ms, "elements_per_s": bp.nb_elem / (vol_ms * 1e-3), "work": grad_work(vol_ms, 1)},
+        "volume_gradient": {"ms": vol_ms, "elements_per_s": bp.nb_elem / (vol_ms * 1e-3), "work": grad_work(vol_ms, 0)},
     }
     sections = set() if args.only_assembly else set(args.sections.split(","))
     if "solve" in sections:
