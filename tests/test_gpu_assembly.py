@@ -9,7 +9,7 @@ import numpy as np
 import pytest
 
 from oracle import oracle as O
-from tests.helpers import all_face_loads, concat_patches, with_inactive
+from tests.helpers import all_face_loads, concat_patches, set_loads, with_inactive
 from yeti_amd.geometry import make_box_patch
 
 pytestmark = pytest.mark.gpu
@@ -177,6 +177,41 @@ def test_load_point_chunks_match_oracle(gpu, p, ng):
     F = sys_linmat_lindef_static(**a)[3]
     F0 = O.oracle_sys_linmat((), kwargs=a)[3]
     assert np.abs(F - F0).max() <= 1e-12 * np.abs(F0).max()
+
+
+@pytest.mark.parametrize("face", [5, 6, 7, 8, 9])
+def test_face_codes_above_six_load_face_six(gpu, face):
+    """The face digit of a load code is 1..9 and every digit above 6 means face 6, as in the oracle:
+    normal loads (types 0 and 4) keep face 6's sign on odd digits too, in F (within 1e-12 of its
+    maximum) and in 2 u^T dF/dX (central differences of u^T F, step 1e-6: rounding 1e-16 / 1e-6 of
+    F and a second-order term, within 1e-6 of the maximum)."""
+    import torch
+    from yeti_amd.assembly import Assembler
+    print("[case] face digit", face, flush=True)
+    bp = make_box_patch(nel=(2, 2, 2), p=2, seed=8)
+    rng = np.random.default_rng(face)
+    nd = np.asfortranarray(rng.uniform(-1, 1, size=(2, bp.nb_cp)))
+    u = rng.standard_normal(3 * bp.nb_cp)
+    target = np.arange(1, bp.nb_elem + 1, dtype=np.int32)
+    for typ in (0, 1, 2, 3, 4):
+        a = set_loads(bp.args, [(10 * face + typ, 1.3, target, [2.0] if typ == 4 else [])], nodal_dist=nd)
+        F0 = O.oracle_sys_linmat((), kwargs=a)[3]
+        asm = Assembler(a)
+        try:
+            F = asm.run_rhs().cpu().numpy()
+            assert np.abs(F - F0).max() <= 1e-12 * np.abs(F0).max(), typ
+            g = asm.load_shape_grad(torch.from_numpy(u).cuda()).cpu().numpy()
+            X = np.ascontiguousarray(np.asarray(a["COORDS3D"]).T).reshape(-1)
+            for i in rng.choice(X.size, 6, replace=False):
+                f = []
+                for h in (1e-6, -1e-6):
+                    Y = X.copy()
+                    Y[i] += h
+                    asm.update_coords(torch.from_numpy(Y).cuda())
+                    f.append(2.0 * float(u @ asm.run_rhs().cpu().numpy()))
+                assert abs((f[0] - f[1]) / 2e-6 - g[i]) <= 1e-6 * np.abs(g).max(), (typ, i)
+        finally:
+            asm.close()
 
 
 @pytest.mark.parametrize("nel", [(1, 1, 1), (3, 2, 1), (13, 11, 16)])

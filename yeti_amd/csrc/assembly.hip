@@ -452,8 +452,9 @@ __global__ void __launch_bounds__(256) elem_rhs_kernel(RhsPatch rp, LoadTable lt
                         const double dS = sqrt(n[0] * n[0] + n[1] * n[1] + n[2] * n[2]);
                         for (int d = 0; d < 3; ++d) f[d] = typ == d + 1 ? wq * dS * fmag : 0.0;
                     } else if (typ == 0 || typ == 4) {
-                        // normal load: the cross product of the face tangents, pointing inwards
-                        const double sg = (face & 1) ? wq * fmag : -wq * fmag;
+                        // normal load: the cross product of the face tangents, pointing inwards;
+                        // codes above face 6 are face 6, as for the points above
+                        const double sg = (face == 1 || face == 3 || face == 5) ? wq * fmag : -wq * fmag;
                         for (int d = 0; d < 3; ++d) f[d] = sg * n[d];
                     }
                 }
