@@ -444,6 +444,36 @@ def test_gradlinelastwork_an_dropin_matches_reference(gpu, name):
     assert np.abs(ge1).max() == 0.0 and np.array_equal(gi1, gi)
 
 
+def test_work_gradients_on_another_stream_keep_their_inputs(gpu):
+    """grad_lin_elast_work on a stream that is still busy returns before its kernels have run: the
+    device copies it made of the arguments (from host tensors, and of the adjoints in column-major
+    order) must not be handed out again before then. Tensors of their sizes are allocated and
+    overwritten on the current stream meanwhile; the result has the bits of a call on the current
+    stream."""
+    import torch
+    from yeti_amd.assembly import Assembler
+    print("[case] work gradients on another stream", flush=True)
+    bp = make_box_patch(nel=(4, 3, 3), p=2, seed=6)
+    n3 = 3 * bp.nb_cp
+    rng = np.random.default_rng(1)
+    sol = torch.from_numpy(rng.standard_normal(n3))
+    adj = torch.from_numpy(rng.standard_normal((3, n3)))
+    asm = Assembler(bp.args)
+    try:
+        g0, e0 = (t.clone() for t in asm.grad_lin_elast_work(sol, adj))
+        torch.cuda.synchronize()
+        side = torch.cuda.Stream()
+        with torch.cuda.stream(side):
+            torch.cuda._sleep(100_000_000)
+        g, e = asm.grad_lin_elast_work(sol, adj, stream=side)
+        junk = [torch.full((m,), 1e30, dtype=torch.float64, device="cuda") for m in (n3, 3 * n3) for _ in range(4)]
+        torch.cuda.synchronize()
+        assert torch.equal(g, g0) and torch.equal(e, e0)
+        assert all(float(t.min()) == 1e30 for t in junk)
+    finally:
+        asm.close()
+
+
 def test_32cube_p2_gradient(gpu):
     """The differentiation workload at its size: 32^3 elements, p = 2 (39,304 control points).
     * gradlinelastwork_an (element-wise gradient kernel, polarised) and the matrix-free MODE 2

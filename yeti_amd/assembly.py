@@ -181,6 +181,9 @@ class Assembler:
                                                        int(nadj), int(bool(compute_wint)), int(bool(compute_wext)),
                                                        C.c_void_p(gi.data_ptr()), C.c_void_p(ge.data_ptr()),
                                                        _stream_handle(stream)))
+        if stream is not None:
+            for t in (sol, adj_cm):   # copies of the arguments: kept until that stream has used them
+                t.record_stream(stream)
         return gi.t(), ge.t()
 
     def strain_energy_grad(self, u, g=None, stream=None):
