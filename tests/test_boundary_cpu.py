@@ -140,6 +140,23 @@ def test_set_up_rejects_out_of_range_ids_before_any_device_call(fn, extra):
     assert rc == _abi.YETI_ERR_INVALID_ARGUMENT and "nb_elem" in msg
 
 
+@pytest.mark.parametrize("p,accepted", [(4, True), (5, True), (8, True), (9, False)])
+def test_set_up_accepts_inactive_patches_of_higher_degree(p, accepted):
+    """A second solid patch of degree 5 to 8 (up to 729 nodes) whose elements are all inactive is
+    part of a model that assembles; with active elements degree 5 is refused, and 1000 nodes are
+    refused always."""
+    from tests.helpers import concat_patches
+    d = concat_patches(make_box_patch(nel=(2, 1, 1), p=2), make_box_patch(nel=(1, 2, 1), p=p))
+    rc, msg, _, _ = _counting_create("yeti_asm_create_in", d, 0)
+    assert rc == (0 if p <= 4 else _abi.YETI_ERR_UNSUPPORTED_DEGREE), msg
+    d["activeElement"] = np.array([1, 1, 0, 0], np.int32)
+    rc, msg, used, _ = _counting_create("yeti_asm_create_in", d, 0)
+    if accepted:
+        assert rc == 0 and used > 0, msg
+    else:
+        assert rc == _abi.YETI_ERR_UNSUPPORTED_DEGREE and "nodes" in msg
+
+
 def test_host_drop_in_rejects_bad_connectivity_without_a_device():
     """The host-buffer drop-in validates before it uploads anything."""
     L = _lib.lib()

@@ -263,7 +263,8 @@ static __device__ inline void cross3(const double *a, const double *b, double *c
     c[2] = a[0] * b[1] - a[1] * b[0];
 }
 
-constexpr int RHS_MAXN = 125;   // (4 + 1)^3: the degrees kernel_available admits
+constexpr int RHS_MAXN = 125;   // (4 + 1)^3: nodes of a loaded element, whose degrees kernel_available admits
+constexpr int PATCH_MAXN = 729; // (8 + 1)^3: nodes of a solid patch, with or without active elements
 
 // Dynamic LDS of elem_rhs_kernel: the element's node coordinates, weights, local indices and CP
 // ids (sized by the patch's node count, so that many elements share a CU).
@@ -2091,7 +2092,7 @@ static int create(const yeti_system_inputs *in, int layout, yeti_asm **out) {
         pd->n_loaded = (int32_t)loaded.size();
         if (e1 == hipSuccess) e1 = pd->loaded.upload(loaded.data(), loaded.size());
         if (e1 != hipSuccess) return fail(set_error(YETI_ERR_DEVICE, "upload patch %d: %s", ip + 1, hipGetErrorString(e1)));
-        if (pd->u1 && pd->nnode > RHS_MAXN)
+        if (pd->u1 && pd->nnode > PATCH_MAXN)
             return fail(set_error(YETI_ERR_UNSUPPORTED_DEGREE, "patch %d: too many nodes", ip + 1));
         woff += (int64_t)nn_geo * pd->nelem;
         ieoff += (int64_t)pd->nnode * pd->nelem;
