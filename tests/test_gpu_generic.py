@@ -218,3 +218,39 @@ def test_gpu_general_kernel_tiles_and_offsets(deg, nel, ng):
             assert np.abs(M[:n].cpu().numpy() - Mo[:n]).max() <= 1e-12 * np.abs(Mo).max()
     finally:
         asm.close()
+
+
+@pytest.mark.gpu
+def test_gpu_general_kernel_beyond_one_launch():
+    """67,109,864 elements of degree 1, 1000 more than the 64-thread workgroups of 2^32 threads
+    (a launch takes fewer and drops the rest without an error): 161 GB of values, every element the same (one set of control points), so
+    each must have the bits of the first one, and the first one the values of a one-element model
+    (1e-12 of their maximum)."""
+    import torch
+    from yeti_amd.assembly import Assembler
+    print("[case] general kernel beyond one launch", flush=True)
+    ne = (1 << 26) + 1000
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 200e9:
+        pytest.skip("needs 200 GB of free device memory")
+    bp = make_box_patch(nel=(1, 1, 1), p=1, seed=9)
+    a = dict(bp.args)
+    one = O.oracle_sys_linmat((), kwargs=a)[0]
+    a.update(IEN=np.tile(a["IEN"], ne), weight=np.tile(a["weight"], ne), activeElement=np.ones(ne, np.int32),
+             Nijk=np.asfortranarray(np.broadcast_to(a["Nijk"], (3, ne))), nb_elem_patch=np.array([ne], np.int32),
+             nb_elem=ne, nb_data=300.0 * ne)
+    asm = Assembler(a)
+    del a
+    try:
+        K = torch.empty(asm.nb_data, dtype=torch.float64, device="cuda")
+        K.fill_(float("nan"))
+        asm.run_values(K)
+        rows = K.view(ne, 300)
+        assert np.abs(rows[0].cpu().numpy() - one).max() <= 1e-12 * np.abs(one).max()
+        first = rows[0].clone()
+        for i0 in range(0, ne, 1 << 21):
+            assert bool((rows[i0:i0 + (1 << 21)] == first).all()), i0
+    finally:
+        asm.close()
+        del K, rows
+        torch.cuda.empty_cache()

@@ -461,43 +461,44 @@ static size_t gen_smem_bytes(int nn) {
            (MODE == 1 ? sizeof(uint16_t) * (size_t)((gen_round_entries<NT>(nn) + 7) / 8 * 8) : 0);
 }
 
-template <int NT>
-static void launch_nt(const GenArgs &ga, bool mass, double *Kd, int32_t *Kr, int32_t *Kc, hipStream_t st) {
-    const int nn = ga.n[0] * ga.n[1] * ga.n[2];
-    auto go = [&](auto kern, size_t lds) {
-        hipLaunchKernelGGL(kern, dim3(xcd_grid(ga.n_active)), dim3(Gen<NT, 0>::NTH), lds, st, ga, Kd, Kr, Kc);
-    };
-    if (mass) {
-        if (Kr) go(elem_general_kernel<NT, 1, true>, gen_smem_bytes<NT, 1>(nn));
-        else go(elem_general_kernel<NT, 1, false>, gen_smem_bytes<NT, 1>(nn));
-    } else {
-        if (Kr) go(elem_general_kernel<NT, 0, true>, gen_smem_bytes<NT, 0>(nn));
-        else go(elem_general_kernel<NT, 0, false>, gen_smem_bytes<NT, 0>(nn));
+// A grid holds fewer than 2^32 threads; of a larger one only the remainder is launched, without an
+// error. The elements go in runs below that (p = 1, 64 threads each: 67,108,856 elements, 161 GB of
+// values).
+template <int NT, int MODE>
+static int launch_kind(GenArgs ga, double *Kd, int32_t *Kr, int32_t *Kc, hipStream_t st) {
+    using C = Gen<NT, MODE>;
+    constexpr int64_t MOST = (0xffffffffLL / C::NTH / XCDS * XCDS) / C::PASSES;
+    const size_t lds = gen_smem_bytes<NT, MODE>(ga.n[0] * ga.n[1] * ga.n[2]);
+    const int64_t n = ga.n_active;
+    for (int64_t e0 = 0; e0 < n; e0 += MOST) {
+        ga.n_active = (int32_t)std::min(MOST, n - e0);
+        const dim3 grid(xcd_grid((int64_t)ga.n_active * C::PASSES)), block(C::NTH);
+        if (Kr) hipLaunchKernelGGL((elem_general_kernel<NT, MODE, true>), grid, block, lds, st, ga, Kd, Kr, Kc);
+        else hipLaunchKernelGGL((elem_general_kernel<NT, MODE, false>), grid, block, lds, st, ga, Kd, Kr, Kc);
+        YETI_HIP(hipGetLastError());
+        ga.elems += ga.n_active;
+        ga.offs += ga.n_active;
+        if (ga.geo) ga.geo += ga.n_active * ga.geo_rec;
     }
+    return 0;
+}
+
+template <int NT>
+static int launch_nt(const GenArgs &ga, bool mass, double *Kd, int32_t *Kr, int32_t *Kc, hipStream_t st) {
+    return mass ? launch_kind<NT, 1>(ga, Kd, Kr, Kc, st) : launch_kind<NT, 0>(ga, Kd, Kr, Kc, st);
 }
 
 int launch_elem_general(const GenArgs &ga, bool mass, double *Kd, int32_t *Kr, int32_t *Kc, hipStream_t st) {
     const int nn = ga.n[0] * ga.n[1] * ga.n[2];
-    if (ga.geo && nn == 125 && ga.tab_n == 5 && ga.ng == 5 && !mass) {
-        if (ga.n_active <= 0) return 0;
-        const size_t lds = gen_smem_bytes<8, 0>(nn);
-        const dim3 grid(xcd_grid((int64_t)ga.n_active * Gen<8, 0>::PASSES)), block(Gen<8, 0>::NTH);
-        if (Kr) hipLaunchKernelGGL((elem_general_kernel<8, 0, true>), grid, block, lds, st, ga, Kd, Kr, Kc);
-        else hipLaunchKernelGGL((elem_general_kernel<8, 0, false>), grid, block, lds, st, ga, Kd, Kr, Kc);
-        YETI_HIP(hipGetLastError());
-        return 0;
-    }
+    if (ga.geo && nn == 125 && ga.tab_n == 5 && ga.ng == 5 && !mass) return launch_kind<8, 0>(ga, Kd, Kr, Kc, st);
     if (nn < 1 || nn > GEN_MAXN || ga.tab_n < 1 || ga.tab_n > GEN_MAXP + 1 || ga.ng < 1 || ga.ng > MAX_NG)
         return set_error(YETI_ERR_UNSUPPORTED_DEGREE, "general element kernel: %d nodes, %d points", nn, ga.ng);
-    if (ga.n_active <= 0) return 0;
     switch ((nn + 15) / 16) {
-    case 1: launch_nt<1>(ga, mass, Kd, Kr, Kc, st); break;
-    case 2: launch_nt<2>(ga, mass, Kd, Kr, Kc, st); break;
-    case 3: launch_nt<3>(ga, mass, Kd, Kr, Kc, st); break;
-    default: launch_nt<4>(ga, mass, Kd, Kr, Kc, st); break;
+    case 1: return launch_nt<1>(ga, mass, Kd, Kr, Kc, st);
+    case 2: return launch_nt<2>(ga, mass, Kd, Kr, Kc, st);
+    case 3: return launch_nt<3>(ga, mass, Kd, Kr, Kc, st);
+    default: return launch_nt<4>(ga, mass, Kd, Kr, Kc, st);
     }
-    YETI_HIP(hipGetLastError());
-    return 0;
 }
 
 }  // namespace yeti
