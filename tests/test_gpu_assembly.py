@@ -239,3 +239,37 @@ def test_p3_kernel_runs_and_offsets(gpu, nel):
         V = torch.zeros(n + 1, dtype=torch.float64, device="cuda")
         asm.run_values(V)
         assert torch.equal(V[:n], K[:n]) and float(K[n:].abs().max()) == 0.0
+
+
+def test_right_hand_side_beyond_one_launch(gpu):
+    """2^24 + 5 elements of degree 1 with a body load, 5 more than the 256-thread workgroups of 2^32
+    threads (a launch takes fewer and drops the rest without an error): element e has the control
+    points of group e mod 4096, so F is the one-element model's times the group's element count
+    (added one by one: 4097 roundings, 1e-12 of the maximum)."""
+    import torch
+    from yeti_amd.assembly import Assembler
+    ne, ng = (1 << 24) + 5, 4096
+    print("[case] right-hand side beyond one launch", flush=True)
+    torch.cuda.empty_cache()
+    if torch.cuda.mem_get_info()[0] < 80e9:
+        pytest.skip("needs 80 GB of free device memory")
+    bp = make_box_patch(nel=(1, 1, 1), p=1, seed=9)
+    one = set_loads(bp.args, [(102, -1.5, [1], [0.2, -0.7, 0.4])])
+    F1 = O.oracle_sys_linmat((), kwargs=one)[3]
+    group = np.arange(ne, dtype=np.int32) % ng
+    every = np.arange(1, ne + 1, dtype=np.int32)
+    a = set_loads(bp.args, [(102, -1.5, every, [0.2, -0.7, 0.4])], nodal_dist=np.zeros((1, 8 * ng), order="F"))
+    a.update(IEN=(8 * group[:, None] + one["IEN"][None, :]).ravel(), weight=np.tile(one["weight"], ne),
+             activeElement=np.ones(ne, np.int32), Nijk=np.asfortranarray(np.broadcast_to(one["Nijk"], (3, ne))),
+             nb_elem_patch=np.array([ne], np.int32), nb_elem=ne, nb_data=300.0 * ne, nb_cp=8 * ng, nb_dof_tot=24 * ng,
+             COORDS3D=np.asfortranarray(np.tile(one["COORDS3D"], ng)), ind_dof_free=np.arange(1, 24 * ng + 1, dtype=np.int32),
+             nb_dof_free=24 * ng)
+    asm = Assembler(a)
+    del a, every, group
+    try:
+        F = asm.run_rhs().cpu().numpy().reshape(ng, 24)
+    finally:
+        asm.close()
+    count = np.full(ng, ne // ng)
+    count[:ne % ng] += 1
+    assert np.abs(F - count[:, None] * F1[None, :]).max() <= 1e-12 * np.abs(F).max()

@@ -1937,14 +1937,18 @@ static int run_rhs(yeti_asm *h, double *F, hipStream_t st) {
             rp.U[d] = pd->U[d].p;
             rp.p[d] = pd->p[d];
         }
-        rp.elems = pd->loaded.p;
-        rp.n_loaded = pd->n_loaded;
-        rp.slot0 = pd->slot0;
         rp.ng = pd->ng;
         rp.rho = pd->rho;
         gauss_legendre(pd->ng, rp.g.x, rp.g.w);
-        hipLaunchKernelGGL(elem_rhs_kernel, dim3(pd->n_loaded), dim3(256), rhs_smem_bytes(rp), st, rp, lt, h->rhs_buf.p);
-        YETI_HIP(hipGetLastError());
+        // a grid holds fewer than 2^32 threads: 2^23 elements of 256 per launch
+        constexpr int32_t MOST = 1 << 23;
+        for (int32_t e0 = 0; e0 < pd->n_loaded; e0 += MOST) {
+            rp.elems = pd->loaded.p + e0;
+            rp.n_loaded = std::min(MOST, pd->n_loaded - e0);
+            rp.slot0 = pd->slot0 + e0;
+            hipLaunchKernelGGL(elem_rhs_kernel, dim3(rp.n_loaded), dim3(256), rhs_smem_bytes(rp), st, rp, lt, h->rhs_buf.p);
+            YETI_HIP(hipGetLastError());
+        }
     }
     int blocks = (h->nb_cp + 255) / 256;
     hipLaunchKernelGGL(rhs_gather_kernel, dim3(blocks), dim3(256), 0, st, h->nb_cp, h->F_conc.p,
