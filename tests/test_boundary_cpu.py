@@ -157,6 +157,19 @@ def test_set_up_accepts_inactive_patches_of_higher_degree(p, accepted):
         assert rc == _abi.YETI_ERR_UNSUPPORTED_DEGREE and "nodes" in msg
 
 
+def test_set_up_rejects_more_loaded_elements_than_int32_entries():
+    """A loaded element takes 125 right-hand side entries, which are numbered in int32: 17,179,870
+    loaded elements are refused (their last entries would be negative) before any device call."""
+    ne = (2 ** 31 - 1) // 125 + 1
+    d = dict(make_box_patch(nel=(1, 1, 1), p=1).args)
+    d.update(IEN=np.tile(d["IEN"], ne), weight=np.tile(d["weight"], ne), activeElement=np.ones(ne, np.int32),
+             Nijk=np.asfortranarray(np.broadcast_to(d["Nijk"], (3, ne))), nb_elem_patch=np.array([ne], np.int32),
+             nb_elem=ne, nb_data=300.0 * ne, indDLoad=np.arange(1, ne + 1, dtype=np.int32),
+             load_target_nbelem=np.array([ne], np.int32))
+    rc, msg, _, out = _counting_create("yeti_asm_create_in", d, 0)
+    assert rc == _abi.YETI_ERR_SIZE_OVERFLOW and "loaded elements" in msg and out is None, (rc, msg)
+
+
 def test_host_drop_in_rejects_bad_connectivity_without_a_device():
     """The host-buffer drop-in validates before it uploads anything."""
     L = _lib.lib()

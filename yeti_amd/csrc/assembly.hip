@@ -2079,12 +2079,12 @@ static int create(const yeti_system_inputs *in, int layout, yeti_asm **out) {
         std::vector<int32_t> loaded;
         pd->slot0 = slot;
         if (pd->u1 && !u0) {
-            for (int e = 0; e < pd->nelem; ++e) {
-                if (in->activeElement[eloff + e] != 1) continue;
-                auto &ls = loads_of_elem[eloff + e];
-                if (ls.empty()) continue;
-                loaded.push_back(e);
-                for (int il : ls) elem_loads.push_back(il);
+            for (int e = 0; e < pd->nelem; ++e)
+                if (in->activeElement[eloff + e] == 1 && !loads_of_elem[eloff + e].empty()) loaded.push_back(e);
+            if ((slot + (int64_t)loaded.size()) * RHS_MAXN > INT32_MAX)   // cp_ent holds int32 entries
+                return fail(set_error(YETI_ERR_SIZE_OVERFLOW, "%lld loaded elements", slot + (long long)loaded.size()));
+            for (int32_t e : loaded) {
+                for (int il : loads_of_elem[eloff + e]) elem_loads.push_back(il);
                 elem_loads_ptr.push_back((int32_t)elem_loads.size());
                 for (int a = 0; a < pd->nnode; ++a) {
                     int32_t cp = in->IEN[ieoff + (int64_t)pd->nnode * e + a] - 1;
