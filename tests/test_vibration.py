@@ -163,3 +163,32 @@ def test_gpu_gradient_waves_and_strides(nel, p):
         asm.close()
     go = O.oracle_grad_vibration(d, V, np.array([2e6]))
     assert np.abs(g - go).max() <= 1e-11 * np.abs(go).max()
+
+
+@pytest.mark.gpu
+def test_gpu_gradient_gather_beyond_its_grid():
+    """1.5 million control points, nearly all unused, with 4 modes: 18 million outputs for the
+    gather's 16.8 million threads at most. The used points have the bits of the model without the
+    others, the rest are zero."""
+    import torch
+    from yeti_amd.assembly import Assembler
+    print("[case] gradient gather beyond its grid", flush=True)
+    d = dict(make_box_patch(nel=(2, 2, 1), p=2, seed=9, rho=7.8e-9).args)
+    n, ncp = int(d["nb_cp"]), 1_500_000
+    V = np.random.default_rng(3).standard_normal((4, 3, n))
+    lam = np.linspace(1e6, 4e7, 4)
+    asm = Assembler(d)
+    g = asm.run_vib_grad(V, lam).clone()
+    asm.close()
+    # the used points last: their outputs lie past the grid's threads
+    X = np.zeros((3, ncp), order="F")
+    X[:, ncp - n:] = d["COORDS3D"]
+    d.update(COORDS3D=X, IEN=(d["IEN"] + ncp - n).astype(np.int32), bc_target=(d["bc_target"] + ncp - n).astype(np.int32),
+             nb_cp=ncp, nb_dof_tot=3 * ncp, nb_dof_free=3 * ncp, ind_dof_free=np.arange(1, 3 * ncp + 1, dtype=np.int32),
+             nodal_dist=np.zeros((1, ncp), order="F"))
+    W = torch.zeros(ncp, 3, 4, dtype=torch.float64, device="cuda")
+    W[ncp - n:] = torch.from_numpy(V).cuda().permute(2, 1, 0)
+    asm = Assembler(d)
+    h = asm.run_vib_grad(W.permute(2, 1, 0), lam)
+    asm.close()
+    assert torch.equal(h[:, :, ncp - n:], g) and float(h[:, :, :ncp - n].abs().max()) == 0.0

@@ -1611,23 +1611,24 @@ __global__ void __launch_bounds__(256) grad_gather_kernel(int32_t nb_cp, const i
                                                           const double *__restrict__ mass, double scale, int32_t k0,
                                                           int32_t nk, double *__restrict__ out) {
     constexpr int GU = 8;
-    const int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     const int row = 3 * nf;
-    if (x >= row * (int64_t)nb_cp) return;
-    const int32_t cp = (int32_t)(x / row);
-    const int fm = (int)(x - row * (int64_t)cp), f = fm / 3, m = fm - 3 * f;
-    const double *g = eg + fm;
-    double s = 0.0;
-    const int j1 = ptr[cp + 1];
-    for (int j = ptr[cp]; j < j1; j += GU) {
-        double v[GU];
+    for (int64_t x = (int64_t)blockIdx.x * blockDim.x + threadIdx.x; x < row * (int64_t)nb_cp;
+         x += (int64_t)gridDim.x * blockDim.x) {
+        const int32_t cp = (int32_t)(x / row);
+        const int fm = (int)(x - row * (int64_t)cp), f = fm / 3, m = fm - 3 * f;
+        const double *g = eg + fm;
+        double s = 0.0;
+        const int64_t j1 = ptr[cp + 1];
+        for (int64_t j = ptr[cp]; j < j1; j += GU) {
+            double v[GU];
 #pragma unroll
-        for (int u = 0; u < GU; ++u) v[u] = g[row * (int64_t)ent[min(j + u, j1 - 1)]];
+            for (int u = 0; u < GU; ++u) v[u] = g[row * (int64_t)ent[min(j + u, j1 - 1)]];
 #pragma unroll
-        for (int u = 0; u < GU; ++u) s += j + u < j1 ? v[u] : 0.0;
+            for (int u = 0; u < GU; ++u) s += j + u < j1 ? v[u] : 0.0;
+        }
+        s *= scale;
+        out[(k0 + f) + (int64_t)nk * (m + 3 * (int64_t)cp)] = mass ? s / mass[f] : s;
     }
-    s *= scale;
-    out[(k0 + f) + (int64_t)nk * (m + 3 * (int64_t)cp)] = mass ? s / mass[f] : s;
 }
 
 // the sum-factorised kernel takes max(p) + 1 Gauss points (all degrees the stiffness accepts);
@@ -1802,7 +1803,8 @@ static int run_shape_grad(yeti_asm *h, GradKind kind, const double *f0, const do
                                mass);
             YETI_HIP(hipGetLastError());
         }
-        const unsigned blocks = (unsigned)((3 * gf.nf * (int64_t)h->nb_cp + 255) / 256);
+        // a bounded grid: one of 2^32 threads or more would drop all but the remainder
+        const unsigned blocks = (unsigned)std::min<int64_t>((3 * gf.nf * (int64_t)h->nb_cp + 255) / 256, 65536);
         hipLaunchKernelGGL(grad_gather_kernel, dim3(blocks), dim3(256), 0, st, h->nb_cp, (const int32_t *)h->vib_ptr.p,
                            (const int32_t *)h->vib_ent.p, (const double *)h->vib_eg.p, gf.nf,
                            normalize ? (const double *)mass : (const double *)nullptr, scale, k0, npair, out);
