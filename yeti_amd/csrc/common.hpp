@@ -41,6 +41,14 @@ int validate_system_inputs(const yeti_system_inputs *in, bool require_solid);
 
 typedef double f64x4 __attribute__((ext_vector_type(4)));
 
+// Orders the LDS accesses of a wave's lanes before it against those after it (the hardware keeps a
+// wave's LDS accesses in order, so it costs no instruction; the compiler must not reorder them).
+__device__ __forceinline__ void wave_lds_sync() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
 // Gauss-Legendre rule passed to kernels by value (orders 1..9, as YETI's table).
 constexpr int MAX_NG = 9;
 struct GaussRule {

@@ -157,7 +157,8 @@ elem_p3_kernel(const double *__restrict__ geo, const int64_t *__restrict__ offs,
         f.load(geo + elem_at(0) * REC, lane);
         for (int64_t s = 0;; ++s) {
             // ---- step A ----
-            wl[lane] = f.w;
+            wl[lane] = f.w;   // put reads other lanes' weights
+            wave_lds_sync();
             f64x4 D[4][4];   // [combination][g1, then i2]
             double ck[4], cl[4], c[4][3];
 #pragma unroll
@@ -365,9 +366,7 @@ elem_p3_kernel(const double *__restrict__ geo, const int64_t *__restrict__ offs,
             if (prev >= 0) store(CS{}, CN{}, prev);
 #pragma unroll
             for (int c = 0; c < 3; ++c) dof[3 * lane + c] = d + c;
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            wave_lds_sync();
             __syncthreads();
             store(C0{}, CS{}, base);
             prev = base;

@@ -82,12 +82,6 @@ struct Grad {
     static constexpr int NEL = NA + NB + NNP;                 // + the node weights
 };
 
-__device__ __forceinline__ void wave_lds_sync() {
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-}
-
 template <int N, int Q, int KIND>
 __global__ void __launch_bounds__((64 * Grad<N, Q>::WPB)) __attribute__((amdgpu_waves_per_eu(N == 5 ? 1 : 3)))
 shape_grad_kernel(GradArgs ga) {
