@@ -428,6 +428,7 @@ row_values_kernel(int32_t nb_cp, int32_t upper, int32_t sstride, const int64_t *
     const int64_t b0 = bptr[I];
     const int nb = (int)(bptr[I + 1] - b0), jd = bdiag[I], nu = nb - jd;
     for (int x = lane; x < 9 * nu; x += 64) acc[x] = 0.0;
+    wave_lds_sync();
     const int64_t k1 = iptr[I + 1];
     int64_t k = iptr[I], code = k < k1 ? irow[k] : 0, next = k + 1 < k1 ? irow[k + 1] : 0;
     int x0 = 0;
@@ -484,6 +485,7 @@ row_values_kernel(int32_t nb_cp, int32_t upper, int32_t sstride, const int64_t *
                 p[3 * kk + ll] += kk == ll ? 2.0 * v[u] : v[u];
                 if (kk != ll) p[3 * ll + kk] += v[u];
             }
+            wave_lds_sync();   // the next step's lanes may add to these addresses
         }
 #pragma unroll
         for (int u = 0; u < RG; ++u) v[u] = w[u];
@@ -493,9 +495,7 @@ row_values_kernel(int32_t nb_cp, int32_t upper, int32_t sstride, const int64_t *
         code = cn;
         x0 = xn;
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+    wave_lds_sync();
     // row I: 3 nu consecutive values for each dof
     for (int kk = 0; kk < 3; ++kk) {
         double *o = vals + 9 * b0 + 3LL * kk * nb + 3 * jd;
