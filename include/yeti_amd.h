@@ -203,6 +203,12 @@ void    yeti_asm_destroy(yeti_asm *h);
 typedef struct yeti_csr yeti_csr;
 
 int32_t yeti_csr_create(const yeti_asm *h, void *stream, yeti_csr **out);
+/* As yeti_csr_create, with the way yeti_csr_values gathers given: 0 element rows (elements numbered
+ * strictly against their CPs, at most 128 nodes), 1 short rows (at most 16 blocks J >= I each), 2 blocks
+ * J >= I, 3 every block, -1 what suits the model; YETI_ERR_INVALID_ARGUMENT when the model does not
+ * allow it. All give the same bits. yeti_csr_values_kind: the way taken. */
+int32_t yeti_csr_create_as(const yeti_asm *h, int32_t kind, void *stream, yeti_csr **out);
+int32_t yeti_csr_values_kind(const yeti_csr *c);
 int64_t yeti_csr_nnz(const yeti_csr *c);
 int32_t yeti_csr_nrows(const yeti_csr *c);
 const int64_t *yeti_csr_rowptr(const yeti_csr *c);   /* device, [nrows + 1] */

@@ -58,29 +58,71 @@ def test_csr_matches_scipy(gpu, nel, p):
     _check_case(bp.args, "csr box %s p=%d" % (nel, p))
 
 
-@pytest.mark.parametrize("nel,p,relabel", [((9, 8, 7), 1, False), ((9, 8, 7), 1, True), ((6, 5, 5), 2, False),
-                                           ((6, 5, 5), 2, True), ((3, 2, 1), 2, True), ((3, 4, 3), 3, True),
-                                           ((3, 4, 3), 3, False), ((3, 2, 2), 4, False)])
-def test_csr_values_by_rows_and_by_blocks(gpu, nel, p, relabel):
+def _relabelled(a, seed):
+    """The model with its control points numbered at random."""
+    ncp = int(a["nb_cp"])
+    new = np.random.default_rng(seed).permutation(ncp)          # old id -> new id, 0-based
+    X = np.empty_like(a["COORDS3D"])
+    X[:, new] = a["COORDS3D"]
+    a["COORDS3D"] = np.asfortranarray(X)
+    a["IEN"] = (new[a["IEN"] - 1] + 1).astype(np.int32)
+    a["bc_target"] = (new[a["bc_target"] - 1] + 1).astype(np.int32)
+    free = a["ind_dof_free"][:a["nb_dof_free"]].astype(np.int64) - 1
+    ind = np.zeros_like(a["ind_dof_free"])
+    ind[:free.size] = np.sort(3 * new[free // 3] + free % 3) + 1
+    a["ind_dof_free"] = ind
+    return a
+
+
+ROWS, SHORT, LIST, EVERY = 0, 1, 2, 3
+
+
+@pytest.mark.parametrize("nel,p,relabel,kinds", [
+    ((9, 8, 7), 1, False, (ROWS, SHORT, LIST, EVERY)), ((9, 8, 7), 1, True, (LIST, EVERY)),
+    ((6, 5, 5), 2, False, (ROWS, LIST, EVERY)), ((6, 5, 5), 2, True, (LIST, EVERY)),
+    ((3, 2, 1), 2, True, (LIST, EVERY)), ((3, 4, 3), 3, True, (LIST, EVERY)),
+    ((3, 4, 3), 3, False, (ROWS, LIST, EVERY)), ((3, 2, 2), 4, False, (ROWS, LIST, EVERY))])
+def test_csr_values_by_rows_and_by_blocks(gpu, nel, p, relabel, kinds):
     """The ways the values are gathered: whole element rows (elements numbered against their
-    control points, rows long enough, one or two slots per lane), and block by block (short rows,
-    16 to 64 lanes each; control points numbered at random), with inactive elements."""
+    control points, one slot per lane, two at p = 4), 16 lanes per short row, the listed blocks
+    J >= I with their transposes, and every block by itself, with inactive elements and control
+    points in order or numbered at random. Against scipy in the way the model takes by itself; the
+    others have its bits, and the ways the model does not allow are refused."""
+    import torch
+    from yeti_amd._lib import YetiError
+    from yeti_amd.solver import StiffnessCSR
     a = dict(make_box_patch(nel=nel, p=p, seed=4 + p).args)
     a["activeElement"] = a["activeElement"].copy()
     a["activeElement"][[0, -1]] = 0
     if relabel:
-        ncp = int(a["nb_cp"])
-        new = np.random.default_rng(p).permutation(ncp)          # old id -> new id, 0-based
-        X = np.empty_like(a["COORDS3D"])
-        X[:, new] = a["COORDS3D"]
-        a["COORDS3D"] = np.asfortranarray(X)
-        a["IEN"] = (new[a["IEN"] - 1] + 1).astype(np.int32)
-        a["bc_target"] = (new[a["bc_target"] - 1] + 1).astype(np.int32)
-        free = a["ind_dof_free"][:a["nb_dof_free"]].astype(np.int64) - 1
-        ind = np.zeros_like(a["ind_dof_free"])
-        ind[:free.size] = np.sort(3 * new[free // 3] + free % 3) + 1
-        a["ind_dof_free"] = ind
-    _check_case(a, "csr %s p=%d relabel=%s" % (nel, p, relabel))
+        a = _relabelled(a, p)
+    asm, csr, K, vals, _ = _check_case(a, "csr %s p=%d relabel=%s" % (nel, p, relabel))
+    for kind in (ROWS, SHORT, LIST, EVERY):
+        if kind not in kinds and not (kind == SHORT and relabel and p == 1):
+            with pytest.raises(YetiError):
+                StiffnessCSR(asm, kind=kind)
+        elif kind in kinds:
+            other = StiffnessCSR(asm, kind=kind)
+            assert other.kind == kind and torch.equal(other.values(K), vals), kind
+
+
+@pytest.mark.parametrize("nel,p,relabel,kind", [
+    ((9, 8, 7), 1, False, SHORT), ((9, 8, 7), 1, True, EVERY), ((8, 8, 8), 2, False, LIST), ((16, 15, 16), 2, False, ROWS),
+    ((16, 15, 16), 2, True, LIST), ((12, 12, 11), 3, False, ROWS), ((8, 8, 8), 4, False, LIST), ((18, 18, 17), 4, False, ROWS),
+    (((40, 8, 8), (2, 2, 2)), (1, 4), False, LIST)])
+def test_csr_way_taken(gpu, nel, p, relabel, kind):
+    """Which way a model takes: element rows from enough rows on (more at p = 4), 16 lanes per row
+    at p = 1 unless a patch of higher degree has longer rows, every block where short rows are
+    numbered at random, the list of blocks J >= I otherwise."""
+    from yeti_amd.assembly import Assembler
+    from yeti_amd.solver import StiffnessCSR
+    if isinstance(p, tuple):
+        a = concat_patches(make_box_patch(nel=nel[0], p=p[0]), make_box_patch(nel=nel[1], p=p[1]))
+    else:
+        a = dict(make_box_patch(nel=nel, p=p).args)
+    if relabel:
+        a = _relabelled(a, 7)
+    assert StiffnessCSR(Assembler(a)).kind == kind
 
 
 def test_csr_multipatch(gpu):

@@ -42,6 +42,8 @@ SIGNATURES = {
     "yeti_asm_kernel_times": (C.c_int32, [C.c_void_p, C.c_void_p, C.c_int32, C.POINTER(C.c_int32)]),
     "yeti_asm_destroy": (None, [C.c_void_p]),
     "yeti_csr_create": (C.c_int32, [C.c_void_p, C.c_void_p, C.POINTER(C.c_void_p)]),
+    "yeti_csr_create_as": (C.c_int32, [C.c_void_p, C.c_int32, C.c_void_p, C.POINTER(C.c_void_p)]),
+    "yeti_csr_values_kind": (C.c_int32, [C.c_void_p]),
     "yeti_csr_nnz": (C.c_int64, [C.c_void_p]),
     "yeti_csr_nrows": (C.c_int32, [C.c_void_p]),
     "yeti_csr_rowptr": (C.c_void_p, [C.c_void_p]),

@@ -5,12 +5,14 @@
 // (overlay/iga_model.py:391-395; benchs/volume_force/test_volume_force_3d.py:69-79).
 //
 // Pattern (once, from the resident connectivity): CP -> (element, local node) incidence,
-// sorted by element; per CP row the sorted set of CPs sharing an element (3x3 block pattern);
-// per block J >= I the list of element contributions in ascending element order. Values (every
-// assembly): one thread per such block sums its contributions read from the COO values in that fixed
-// order -- deterministic, no floating-point atomics -- and writes the block and its transpose. Scalar CSR: dof row 3 I + k holds, for each
-// block column J of CP row I (ascending), the columns 3 J, 3 J + 1, 3 J + 2: scipy's canonical
-// layout of the structural pattern.
+// sorted by element; per CP row the sorted set of CPs sharing an element (3x3 block pattern).
+// Values (every assembly): a block's contributions are read from the COO values and summed in
+// ascending element order -- deterministic, no floating-point atomics. Two ways, chosen at creation
+// (CsrValues): the element rows of a CP streamed whole (row_values_kernel), or block by block from a list
+// of each block's contributions (csr_values_kernel). Blocks J >= I are summed and written twice, as (I, J)
+// and, transposed, as (J, I); short rows of a model numbered at random sum every block. Scalar CSR: dof
+// row 3 I + k holds, for each block column J of CP row I (ascending), the columns 3 J, 3 J + 1, 3 J + 2:
+// scipy's canonical layout of the structural pattern.
 #include <algorithm>
 #include <vector>
 
@@ -31,6 +33,14 @@ struct AsmView {
 int asm_view(const yeti_asm *h, AsmView *v);
 }  // namespace yeti
 
+// how the values are gathered
+enum CsrValues {
+    CSR_ROWS,    // element rows
+    CSR_SHORT,   // blocks J >= I, 16 lanes per CP row
+    CSR_LIST,    // blocks J >= I, one thread each
+    CSR_EVERY,   // every block, one thread each
+};
+
 struct yeti_csr {
     int32_t nb_cp = 0;
     int64_t nblocks = 0;                 // 3x3 blocks
@@ -38,14 +48,18 @@ struct yeti_csr {
     yeti::DevBuf<int32_t> bcol;          // [nblocks]
     yeti::DevBuf<int32_t> bdiag;         // [nb_cp] place of the diagonal block in its row (the row's length: none)
     yeti::DevBuf<uint16_t> mirror;       // [nblocks] block (I, J), J > I: place of block (J, I) in row J
-    // values by element rows (row_values_kernel), when upper > 0:
+    CsrValues kind = CSR_LIST;
+    // CSR_ROWS:
     int32_t upper = 0;                   // most blocks J >= I of a row
     int32_t sstride = 0;                 // slots per incidence
     yeti::DevBuf<int64_t> iptr;          // [nb_cp + 1] incidences of each CP
     yeti::DevBuf<int64_t> irow;          // (COO position of the element's row of a << 10) | a
     yeti::DevBuf<uint16_t> slots;        // [incidence][b]: place of block (I, J_b) after the diagonal, b <= a
-    // values by blocks (csr_values_kernel) otherwise:
-    yeti::DevBuf<int64_t> cptr;          // [nblocks + 1] contribution offsets (blocks J >= I)
+    // otherwise:
+    int64_t nlist = 0;                   // listed blocks, row by row (CSR_LIST: J >= I; else all)
+    yeti::DevBuf<int64_t> uptr;          // [nb_cp + 1] CSR_LIST: first listed block of each row (else bptr)
+    yeti::DevBuf<int32_t> urow;          // [nlist] CP row of each (CSR_SHORT: none)
+    yeti::DevBuf<int64_t> cptr;          // [nlist + 1] contribution offsets
     yeti::DevBuf<int64_t> contrib;       // (COO position << 2) | kind
     yeti::DevBuf<int64_t> rowptr;        // scalar CSR [3 nb_cp + 1]
     yeti::DevBuf<int32_t> colind;        // scalar CSR [9 nblocks]
@@ -106,12 +120,14 @@ __global__ void scan_block_kernel(const T *in, int64_t n, int64_t *out, int64_t 
         __syncthreads();
     }
     if (i < n) out[i] = s[threadIdx.x] - v;
+    if (i == n - 1) out[n] = s[threadIdx.x];
     if (threadIdx.x == 1023) bsum[blockIdx.x] = s[1023];
 }
 
 __global__ void scan_add_kernel(int64_t *out, int64_t n, const int64_t *boff) {
     int64_t i = (int64_t)blockIdx.x * 1024 + threadIdx.x;
     if (i < n) out[i] += boff[blockIdx.x];
+    if (i == n - 1) out[n] += boff[blockIdx.x];
 }
 
 // exclusive scan of n values into out[0..n], out[n] = total. Host-driven recursion.
@@ -133,14 +149,11 @@ static int exclusive_scan(const T *in, int64_t n, int64_t *out, hipStream_t st) 
         hipLaunchKernelGGL(scan_add_kernel, dim3((unsigned)nb), dim3(1024), 0, st, out, n, boff.p);
         YETI_HIP(hipGetLastError());
     }
-    // total = last offset + last count
-    int64_t last_off = 0;
-    T last_in{};
-    YETI_HIP(hipMemcpyAsync(&last_off, out + n - 1, sizeof(int64_t), hipMemcpyDeviceToHost, st));
-    YETI_HIP(hipMemcpyAsync(&last_in, in + n - 1, sizeof(T), hipMemcpyDeviceToHost, st));
-    YETI_HIP(hipStreamSynchronize(st));
-    int64_t total = last_off + (int64_t)last_in;
-    YETI_HIP(hipMemcpyAsync(out + n, &total, sizeof(int64_t), hipMemcpyHostToDevice, st));
+    return 0;
+}
+
+static int read_back(void *host, const void *dev, size_t bytes, hipStream_t st) {
+    YETI_HIP(hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st));
     YETI_HIP(hipStreamSynchronize(st));
     return 0;
 }
@@ -228,17 +241,22 @@ __global__ void __launch_bounds__(256) row_pattern_kernel(int32_t nb_cp, const i
     }
 }
 
-// Per row: count (pass 1) or write (pass 2) the contributions of each block J >= I, in element order.
+// Per row: count (pass 1) or write (pass 2) the contributions of its blocks from place `first` on (bdiag, or
+// 0 when null), in element order; block i of the row is number lptr[row] + i of the list, or
+// lptr[row] + i - first when `dense`.
 // kind 0: block (a, b) stored as is (a < b); 1: stored as (b, a) (a > b, transpose);
 // 2: diagonal block (a == b), stored as its 6 upper entries with the diagonal halved.
 template <bool FILL>
 __global__ void __launch_bounds__(64) contrib_kernel(int32_t nb_cp, const int64_t *inc_ptr, const int64_t *inc,
                                                      PatchIen pi, const int64_t *bptr, const int32_t *bcol,
+                                                     const int32_t *bdiag, const int64_t *lptr, bool dense,
                                                      int32_t *bcount, const int64_t *cptr, int64_t *contrib) {
     __shared__ int32_t cur[1024];
     const int row = blockIdx.x, lane = threadIdx.x;
     if (row >= nb_cp) return;
     const int64_t b0 = bptr[row];
+    const int first = bdiag ? bdiag[row] : 0;
+    const int64_t u0 = lptr[row] - (dense ? first : 0);
     const int nb = (int)(bptr[row + 1] - b0);
     if (nb > 1024) return;      // rejected by the pattern pass (overflow flag)
     for (int i = lane; i < nb; i += 64) cur[i] = 0;
@@ -252,12 +270,12 @@ __global__ void __launch_bounds__(64) contrib_kernel(int32_t nb_cp, const int64_
         const int32_t *ie = pi.ien[patch] + (int64_t)nn * e;
         for (int b = lane; b < nn; b += 64) {
             int32_t J = ie[b] - 1;
-            if (J < row) continue;
             int lo = 0, hi = nb - 1;       // binary search of J among the row's sorted columns
             while (lo < hi) {
                 int mid = (lo + hi) >> 1;
                 if (bcol[b0 + mid] < J) lo = mid + 1; else hi = mid;
             }
+            if (lo < first) continue;
             // one contribution per (element, block): no two lanes hit the same block here
             int slot = cur[lo]++;
             if (FILL) {
@@ -265,13 +283,39 @@ __global__ void __launch_bounds__(64) contrib_kernel(int32_t nb_cp, const int64_
                 if (a < b) code = ((base + 9LL * b * (b - 1) / 2 + 6LL * b + 9LL * a) << 2) | 0;
                 else if (a > b) code = ((base + 9LL * a * (a - 1) / 2 + 6LL * a + 9LL * b) << 2) | 1;
                 else code = ((base + 9LL * a * (a - 1) / 2 + 6LL * a + 9LL * a) << 2) | 2;
-                contrib[cptr[b0 + lo] + slot] = code;
+                contrib[cptr[u0 + lo] + slot] = code;
             }
         }
         __syncthreads();
     }
     if (!FILL)
-        for (int i = lane; i < nb; i += 64) bcount[b0 + i] = cur[i];
+        for (int i = (dense ? first : 0) + lane; i < nb; i += 64) bcount[u0 + i] = cur[i];
+}
+
+// Number of blocks J >= I per row; flags[0]: the most of a row.
+__global__ void __launch_bounds__(256) upper_count_kernel(int32_t nb_cp, const int64_t *bptr, const int32_t *bdiag,
+                                                          int32_t *count, int32_t *flags) {
+    const int64_t I = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    int n = 0;
+    if (I < nb_cp) count[I] = n = (int32_t)(bptr[I + 1] - bptr[I]) - bdiag[I];
+    for (int o = 32; o > 0; o >>= 1) n = max(n, __shfl_xor(n, o, 64));
+    if ((threadIdx.x & 63) == 0) atomicMax(&flags[0], n);
+}
+
+// flags[1]: set when local nodes of an active element are not numbered strictly against their CPs
+__global__ void __launch_bounds__(256) order_kernel(const int32_t *ien, const int32_t *elems, int n_active, int nn,
+                                                    int32_t *flags) {
+    const int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+    if (t >= (int64_t)n_active * nn || t % nn == 0) return;
+    const int32_t *ie = ien + (int64_t)nn * elems[t / nn] + t % nn;
+    if (ie[-1] <= ie[0]) flags[1] = 1;   // every writer writes the same
+}
+
+// CP row of each listed block
+__global__ void __launch_bounds__(256) list_rows_kernel(int32_t nb_cp, const int64_t *lptr, int32_t *urow) {
+    const int64_t I = (int64_t)blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (I >= nb_cp) return;
+    for (int64_t x = lptr[I] + (threadIdx.x & 63); x < lptr[I + 1]; x += 64) urow[x] = (int32_t)I;
 }
 
 // The diagonal block's place in each row, and for every block above it the place of its transpose.
@@ -293,6 +337,28 @@ __global__ void __launch_bounds__(256) mirror_kernel(int32_t nb_cp, const int64_
     const int jd = place(I, (int32_t)I), nb = (int)(bptr[I + 1] - bptr[I]);
     if (lane == 0) bdiag[I] = jd;
     for (int j = jd + lane; j < nb; j += 64) mirror[bptr[I] + j] = (uint16_t)place(bcol[bptr[I] + j], (int32_t)I);
+}
+
+// Of the blocks above the diagonal of some rows (one per workgroup, spread over the model): flags[2] their
+// number, flags[3] how many have their transpose right after that of the block in the row before.
+__global__ void __launch_bounds__(64) adjacent_kernel(int32_t nb_cp, const int64_t *bptr, const int32_t *bcol,
+                                                      const int32_t *bdiag, const uint16_t *mirror, int32_t *flags) {
+    const int64_t I = (int64_t)blockIdx.x * nb_cp / gridDim.x, b0 = bptr[I];
+    const int nb = (int)(bptr[I + 1] - b0);
+    int n = 0, adj = 0;
+    for (int j = bdiag[I] + 1 + threadIdx.x; j < nb; j += 64) {
+        const int jm = mirror[b0 + j];
+        ++n;
+        if (jm > 0 && bcol[bptr[bcol[b0 + j]] + jm - 1] == I - 1) ++adj;
+    }
+    for (int o = 32; o > 0; o >>= 1) {
+        n += __shfl_xor(n, o, 64);
+        adj += __shfl_xor(adj, o, 64);
+    }
+    if (threadIdx.x == 0) {
+        atomicAdd(&flags[2], n);
+        atomicAdd(&flags[3], adj);
+    }
 }
 
 __global__ void scalar_pattern_kernel(int32_t nb_cp, const int64_t *bptr, const int32_t *bcol,
@@ -318,89 +384,100 @@ __global__ void scalar_pattern_kernel(int32_t nb_cp, const int64_t *bptr, const 
 }
 
 // ---- values ------------------------------------------------------------------------------
-// LPR lanes per CP row I, each on a block J >= I (its contributions summed in element order), written
-// as block (I, J) and, transposed, as (J, I): each COO value is read once. Local nodes are numbered
-// against the CPs, so a block above the diagonal mostly holds a > b and lies in the element's row of a:
-// its neighbours' contributions are next to it and the lanes read whole cache lines, where the blocks
-// below the diagonal would take 72 bytes out of every line pair. A contribution is read in five loads,
-// UC of them in flight. Each XCD takes one run of rows, so that the transposed blocks of neighbouring
-// rows meet in its L2. 45x40x33 p = 3: 5.35 ms (21.5 GB fetched), against 7.72 ms with one thread for
-// every block, found by binary search; 100x60x60 p = 1, which row_values_kernel does not take,
-// 0.98 -> 0.85 ms with the product.
+// CSR_SHORT: SHORT_ROW lanes per CP row, one on each of its blocks J >= I (at most SHORT_ROW, p = 1: 14);
+// else one thread per listed block (I, J). A block's contributions are summed in element order, UC of
+// them in flight. Blocks J >= I are written also, transposed, as (J, I), so that each COO value is read
+// once; each XCD takes one run of the list, so that the transposed blocks of neighbouring rows meet in
+// its L2. CSR_EVERY lists every block: with control points numbered at random the transposes
+// are 24-byte pieces of separate lines, which costs more than reading a short row's two or three
+// contributions twice (random numbering, 72^3 p = 1: 1626 us mirrored, 892 us by itself; p = 2 at 34^3
+// 882 us mirrored, 1115 us by itself). Blocks are dealt one by one, not row by row: rows differ in their
+// blocks J >= I (random numbering: from none to all), and a small model has more blocks than lanes
+// (against 64 lanes per row: 4^3 p = 4 111 -> 38 us, 8^3 p = 4 numbered at random 851 -> 222 us).
+constexpr int SHORT_ROW = 16;
+
 typedef double f64x2u __attribute__((ext_vector_type(2), aligned(8)));
 
-template <int LPR>
-__global__ void __launch_bounds__(256) csr_values_kernel(int32_t nb_cp, const int64_t *__restrict__ bptr,
-                                                         const int32_t *__restrict__ bcol,
-                                                         const int32_t *__restrict__ bdiag,
-                                                         const uint16_t *__restrict__ mirror,
-                                                         const int64_t *__restrict__ cptr,
-                                                         const int64_t *__restrict__ contrib,
-                                                         const double *__restrict__ Kdata,
-                                                         double *__restrict__ vals) {
+template <int VT, int KIND>
+__global__ void __launch_bounds__(VT) csr_values_kernel(int64_t nitem, const int64_t *__restrict__ lptr,
+                                                        const int32_t *__restrict__ urow,
+                                                        const int64_t *__restrict__ bptr,
+                                                        const int32_t *__restrict__ bcol,
+                                                        const int32_t *__restrict__ bdiag,
+                                                        const uint16_t *__restrict__ mirror,
+                                                        const int64_t *__restrict__ cptr,
+                                                        const int64_t *__restrict__ contrib,
+                                                        const double *__restrict__ Kdata,
+                                                        double *__restrict__ vals) {
     constexpr int UC = 2;
-    constexpr int RPB = 256 / LPR;   // rows per workgroup
-    const int lane = threadIdx.x % LPR;
-    const int64_t I = xcd_element(blockIdx.x, ((int64_t)nb_cp + RPB - 1) / RPB) * RPB + threadIdx.x / LPR;
-    if (I >= nb_cp) return;
+    constexpr bool MIRROR = KIND != CSR_EVERY;
+    int64_t x = xcd_element(blockIdx.x, (nitem + VT - 1) / VT) * VT + threadIdx.x;
+    if (x >= nitem) return;
+    const int32_t I = KIND == CSR_SHORT ? (int32_t)(x / SHORT_ROW) : urow[x];
     const int64_t b0 = bptr[I];
     const int nb = (int)(bptr[I + 1] - b0);
-    for (int j = bdiag[I] + lane; j < nb; j += LPR) {
-        double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};   // v[k][l] = v[3k + l]
-        const int32_t J = bcol[b0 + j];
-        const int jm = mirror[b0 + j];
-        const int64_t c1 = cptr[b0 + j + 1];
-        for (int64_t c = cptr[b0 + j]; c < c1; c += UC) {
-            double s[UC][9];
-            int kind[UC];
+    int j;
+    if (KIND == CSR_SHORT) {
+        j = bdiag[I] + (int)(x % SHORT_ROW);
+        if (j >= nb) return;
+        x = b0 + j;
+    } else {
+        j = (int)(x - lptr[I]) + (KIND == CSR_LIST ? bdiag[I] : 0);
+    }
+    double v[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};   // v[k][l] = v[3k + l]
+    const int32_t J = MIRROR ? bcol[b0 + j] : 0;
+    const int jm = MIRROR ? mirror[b0 + j] : 0;
+    const int64_t c1 = cptr[x + 1];
+    for (int64_t c = cptr[x]; c < c1; c += UC) {
+        double s[UC][9];
+        int kind[UC];
 #pragma unroll
-            for (int u = 0; u < UC; ++u) {
-                const int64_t code = contrib[min(c + u, c1 - 1)];
-                kind[u] = c + u < c1 ? (int)(code & 3) : 3;
-                const double *p = Kdata + (code >> 2);
-                f64x2u t[4] = {};
-                t[0] = *reinterpret_cast<const f64x2u *>(p);
-                t[1] = *reinterpret_cast<const f64x2u *>(p + 2);
-                t[2] = *reinterpret_cast<const f64x2u *>(p + 4);
-                s[u][8] = 0.0;
-                if ((code & 3) != 2) {   // a diagonal block has six entries
-                    t[3] = *reinterpret_cast<const f64x2u *>(p + 6);
-                    s[u][8] = p[8];
-                }
-#pragma unroll
-                for (int x = 0; x < 8; ++x) s[u][x] = t[x / 2][x % 2];
+        for (int u = 0; u < UC; ++u) {
+            const int64_t code = contrib[min(c + u, c1 - 1)];
+            kind[u] = c + u < c1 ? (int)(code & 3) : 3;
+            const double *p = Kdata + (code >> 2);
+            f64x2u t[4] = {};
+            t[0] = *reinterpret_cast<const f64x2u *>(p);
+            t[1] = *reinterpret_cast<const f64x2u *>(p + 2);
+            t[2] = *reinterpret_cast<const f64x2u *>(p + 4);
+            s[u][8] = 0.0;
+            if ((code & 3) != 2) {   // a diagonal block has six entries
+                t[3] = *reinterpret_cast<const f64x2u *>(p + 6);
+                s[u][8] = p[8];
             }
 #pragma unroll
-            for (int u = 0; u < UC; ++u) {
-                const double *q = s[u];
-                if (kind[u] < 2) {   // stored (k, l) at q[k + 3 l]; kind 1: the transpose of the stored block
-                    const bool tr = kind[u] == 1;
+            for (int y = 0; y < 8; ++y) s[u][y] = t[y / 2][y % 2];
+        }
 #pragma unroll
-                    for (int k = 0; k < 3; ++k)
+        for (int u = 0; u < UC; ++u) {
+            const double *q = s[u];
+            if (kind[u] < 2) {   // stored (k, l) at q[k + 3 l]; kind 1: the transpose of the stored block
+                const bool tr = kind[u] == 1;
 #pragma unroll
-                        for (int l = 0; l < 3; ++l) v[3 * k + l] += tr ? q[l + 3 * k] : q[k + 3 * l];
-                } else if (kind[u] == 2) {   // diagonal block: side + side^T, (0,0) (0,1) (1,1) (0,2) (1,2) (2,2)
-                    v[0] += 2.0 * q[0]; v[4] += 2.0 * q[2]; v[8] += 2.0 * q[5];
-                    v[1] += q[1]; v[3] += q[1];
-                    v[2] += q[3]; v[6] += q[3];
-                    v[5] += q[4]; v[7] += q[4];
-                }
+                for (int k = 0; k < 3; ++k)
+#pragma unroll
+                    for (int l = 0; l < 3; ++l) v[3 * k + l] += tr ? q[l + 3 * k] : q[k + 3 * l];
+            } else if (kind[u] == 2) {   // diagonal block: side + side^T, (0,0) (0,1) (1,1) (0,2) (1,2) (2,2)
+                v[0] += 2.0 * q[0]; v[4] += 2.0 * q[2]; v[8] += 2.0 * q[5];
+                v[1] += q[1]; v[3] += q[1];
+                v[2] += q[3]; v[6] += q[3];
+                v[5] += q[4]; v[7] += q[4];
             }
         }
-        double *o = vals + 9 * b0 + 3 * j;
+    }
+    double *o = vals + 9 * b0 + 3 * j;
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+#pragma unroll
+        for (int l = 0; l < 3; ++l) o[3LL * k * nb + l] = v[3 * k + l];
+    if (MIRROR && J != I) {
+        const int64_t m0 = bptr[J];
+        const int mb = (int)(bptr[J + 1] - m0);
+        o = vals + 9 * m0 + 3 * jm;
 #pragma unroll
         for (int k = 0; k < 3; ++k)
 #pragma unroll
-            for (int l = 0; l < 3; ++l) o[3LL * k * nb + l] = v[3 * k + l];
-        if (J != I) {
-            const int64_t m0 = bptr[J];
-            const int mb = (int)(bptr[J + 1] - m0);
-            o = vals + 9 * m0 + 3 * jm;
-#pragma unroll
-            for (int k = 0; k < 3; ++k)
-#pragma unroll
-                for (int l = 0; l < 3; ++l) o[3LL * k * mb + l] = v[3 * l + k];
-        }
+            for (int l = 0; l < 3; ++l) o[3LL * k * mb + l] = v[3 * l + k];
     }
 }
 
@@ -517,17 +594,14 @@ row_values_kernel(int32_t nb_cp, int32_t upper, int32_t sstride, const int64_t *
     }
 }
 
-// Per CP row: the element rows and slots of its incidences; flags[0]: most blocks J >= I of a row,
-// flags[1]: set when some element has a CP J_b < I_a with b < a (numbered otherwise).
+// Per CP row: the element rows and slots of its incidences.
 __global__ void __launch_bounds__(64) slot_kernel(int32_t nb_cp, const int64_t *inc_ptr, const int64_t *inc, PatchIen pi,
                                                   const int64_t *bptr, const int32_t *bcol, const int32_t *bdiag,
-                                                  int32_t sstride, int64_t *irow, uint16_t *slots, int32_t *flags) {
+                                                  int32_t sstride, int64_t *irow, uint16_t *slots) {
     const int row = blockIdx.x, lane = threadIdx.x;
     if (row >= nb_cp) return;
     const int64_t b0 = bptr[row];
     const int nb = (int)(bptr[row + 1] - b0), jd = bdiag[row];
-    if (lane == 0) atomicMax(&flags[0], nb - jd);
-    bool other = false;
     for (int64_t k = inc_ptr[row]; k < inc_ptr[row + 1]; ++k) {
         const int64_t en = inc[k];
         const int patch = (int)(en >> 58), ea = (int)((en >> 10) & ((1LL << 48) - 1)), a = (int)(en & 1023);
@@ -536,10 +610,6 @@ __global__ void __launch_bounds__(64) slot_kernel(int32_t nb_cp, const int64_t *
         if (lane == 0) irow[k] = ((pi.offs[patch][ea] + (9LL * a * a + 3LL * a) / 2) << 10) | a;
         for (int b = lane; b <= a; b += 64) {
             const int32_t J = ie[b] - 1;
-            if (J < row || (b < a && J == row)) {
-                other = true;
-                continue;
-            }
             int lo = jd, hi = nb - 1;
             while (lo < hi) {
                 const int mid = (lo + hi) >> 1;
@@ -548,7 +618,6 @@ __global__ void __launch_bounds__(64) slot_kernel(int32_t nb_cp, const int64_t *
             slots[k * sstride + b] = (uint16_t)(lo - jd);
         }
     }
-    if (other) atomicOr(&flags[1], 1);
 }
 
 // ---- SpMV by nodal 3x3 blocks: one wave per CP row ---------------------------------------
@@ -688,7 +757,7 @@ int32_t yeti_csr_drop_zeros(const yeti_csr *c, const double *vals_dev, int64_t *
         hipLaunchKernelGGL(nz_count_kernel, dim3(g), dim3(256), 0, st, nrows, c->rowptr.p, vals_dev, cnt.p);
         YETI_HIP(hipGetLastError());
     }
-    int rc = exclusive_scan<int32_t>(cnt.p, nrows, rowptr_out, st);   // ends with a stream sync
+    int rc = exclusive_scan<int32_t>(cnt.p, nrows, rowptr_out, st);
     if (rc) return rc;
     if (nrows > 0) {
         hipLaunchKernelGGL(nz_compact_kernel, dim3(g), dim3(256), 0, st, nrows, c->rowptr.p, c->colind.p, vals_dev,
@@ -700,9 +769,10 @@ int32_t yeti_csr_drop_zeros(const yeti_csr *c, const double *vals_dev, int64_t *
     return 0;
 }
 
-int32_t yeti_csr_create(const yeti_asm *h, void *stream, yeti_csr **out) {
+int32_t yeti_csr_create_as(const yeti_asm *h, int32_t kind, void *stream, yeti_csr **out) {
     if (!h || !out) return set_error(YETI_ERR_INVALID_ARGUMENT, "null argument");
     *out = nullptr;
+    if (kind < -1 || kind > CSR_EVERY) return set_error(YETI_ERR_INVALID_ARGUMENT, "CSR: no way %d to gather the values", kind);
     hipStream_t st = (hipStream_t)stream;
     AsmView v;
     int rc = asm_view(h, &v);
@@ -722,7 +792,7 @@ int32_t yeti_csr_create(const yeti_asm *h, void *stream, yeti_csr **out) {
         pi.nn[p] = v.nnode[p];
         if (v.nnode[p] > 729) return fail(set_error(YETI_ERR_UNSUPPORTED_DEGREE, "CSR: too many nodes per element"));
     }
-    DevBuf<int32_t> cnt, cursor, rowlen, bcount, oflow;
+    DevBuf<int32_t> cnt, cursor, rowlen, bcount, oflow, flags;
     DevBuf<int64_t> inc_ptr, inc;
     if (cnt.alloc(v.nb_cp) != hipSuccess || cursor.alloc(v.nb_cp) != hipSuccess ||
         inc_ptr.alloc(v.nb_cp + 1) != hipSuccess)
@@ -738,8 +808,7 @@ int32_t yeti_csr_create(const yeti_asm *h, void *stream, yeti_csr **out) {
     }
     if ((rc = exclusive_scan<int32_t>(cnt.p, v.nb_cp, inc_ptr.p, st))) return fail(rc);
     int64_t ninc = 0;
-    if (hipMemcpy(&ninc, inc_ptr.p + v.nb_cp, 8, hipMemcpyDeviceToHost) != hipSuccess)
-        return fail(set_error(YETI_ERR_DEVICE, "CSR: copy failed"));
+    if ((rc = read_back(&ninc, inc_ptr.p + v.nb_cp, 8, st))) return fail(rc);
     if (inc.alloc(std::max<int64_t>(ninc, 1)) != hipSuccess) return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc inc"));
     for (int p = 0; p < v.npatch; ++p) {
         int64_t n = (int64_t)v.n_active[p] * v.nnode[p];
@@ -750,17 +819,16 @@ int32_t yeti_csr_create(const yeti_asm *h, void *stream, yeti_csr **out) {
     hipLaunchKernelGGL(inc_sort_kernel, dim3((v.nb_cp + 255) / 256), dim3(256), 0, st, v.nb_cp, inc_ptr.p, inc.p);
     // block pattern
     if (rowlen.alloc(v.nb_cp) != hipSuccess || c->bptr.alloc(v.nb_cp + 1) != hipSuccess ||
-        oflow.alloc(1) != hipSuccess || hipMemsetAsync(oflow.p, 0, 4, st) != hipSuccess)
+        oflow.alloc(1) != hipSuccess || hipMemsetAsync(oflow.p, 0, 4, st) != hipSuccess ||
+        flags.alloc(4) != hipSuccess || hipMemsetAsync(flags.p, 0, 16, st) != hipSuccess)
         return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc rows"));
     hipLaunchKernelGGL(row_pattern_kernel<false>, dim3((v.nb_cp + 3) / 4), dim3(256), 0, st, v.nb_cp, inc_ptr.p,
                        inc.p, pi, rowlen.p, nullptr, nullptr, oflow.p);
     int32_t of = 0;
-    if (hipMemcpyAsync(&of, oflow.p, 4, hipMemcpyDeviceToHost, st) != hipSuccess || hipStreamSynchronize(st) != hipSuccess)
-        return fail(set_error(YETI_ERR_DEVICE, "CSR: copy failed"));
+    if ((rc = read_back(&of, oflow.p, 4, st))) return fail(rc);
     if (of) return fail(set_error(YETI_ERR_SIZE_OVERFLOW, "CSR: a control point has more than 1024 neighbours"));
     if ((rc = exclusive_scan<int32_t>(rowlen.p, v.nb_cp, c->bptr.p, st))) return fail(rc);
-    if (hipMemcpy(&c->nblocks, c->bptr.p + v.nb_cp, 8, hipMemcpyDeviceToHost) != hipSuccess)
-        return fail(set_error(YETI_ERR_DEVICE, "CSR: copy failed"));
+    if ((rc = read_back(&c->nblocks, c->bptr.p + v.nb_cp, 8, st))) return fail(rc);
     if (c->bcol.alloc(std::max<int64_t>(c->nblocks, 1)) != hipSuccess)
         return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc bcol"));
     hipLaunchKernelGGL(row_pattern_kernel<true>, dim3((v.nb_cp + 3) / 4), dim3(256), 0, st, v.nb_cp, inc_ptr.p,
@@ -770,50 +838,77 @@ int32_t yeti_csr_create(const yeti_asm *h, void *stream, yeti_csr **out) {
         return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc mirror"));
     hipLaunchKernelGGL(mirror_kernel, dim3((v.nb_cp + 3) / 4), dim3(256), 0, st, v.nb_cp, c->bptr.p, c->bcol.p, c->bdiag.p,
                        c->mirror.p);
-    // element rows, when every element is numbered against its CPs and rows are long enough
-    // (csr_values_kernel packs short rows: at p = 1 a run is 36 entries on average)
+    // CSR_ROWS: every element is numbered against its CPs, rows are long enough (at p = 1 a run is 36
+    // entries on average) and there are enough of them to hide that a row is one wave's chain: by rows and
+    // by blocks p = 2 14^3 43.6 and 42.6 us, 15^3 49.2 and 51.7; p = 3 10^3 112 and 96, 11^3 116 and 140;
+    // p = 4 (half the waves per CU) 14^3 1.10 and 0.94 ms, 18^3 1.98 and 1.89, 24^3 4.08 and 4.36.
+    // CSR_EVERY: short rows of which less than a quarter of the transposes follow that of the row before.
     int32_t nn_max = 1;
     for (int p = 0; p < v.npatch; ++p)
         if (v.n_active[p] > 0) nn_max = std::max(nn_max, v.nnode[p]);
     const int64_t mean = (c->nblocks / std::max(v.nb_cp, 1) + 1) / 2;
-    if (mean > 32 && nn_max <= 128) {
-        DevBuf<int32_t> flags;
-        int32_t fl[2] = {0, 1};
+    const bool long_rows = mean > 32 && c->nblocks / 2 >= (nn_max <= 64 ? 1 << 18 : 1 << 21);
+    int32_t fl[4] = {0, 0, 0, 0};
+    hipLaunchKernelGGL(upper_count_kernel, dim3((v.nb_cp + 255) / 256), dim3(256), 0, st, v.nb_cp, c->bptr.p, c->bdiag.p,
+                       rowlen.p, flags.p);
+    for (int p = 0; p < v.npatch && (long_rows || kind == CSR_ROWS); ++p) {
+        const int64_t n = (int64_t)v.n_active[p] * v.nnode[p];
+        if (n == 0) continue;
+        hipLaunchKernelGGL(order_kernel, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, v.ien[p], v.elems[p],
+                           v.n_active[p], v.nnode[p], flags.p);
+    }
+    if (mean <= SHORT_ROW)
+        hipLaunchKernelGGL(adjacent_kernel, dim3(std::min(v.nb_cp, 4096)), dim3(64), 0, st, v.nb_cp, c->bptr.p, c->bcol.p,
+                           c->bdiag.p, c->mirror.p, flags.p);
+    if ((rc = read_back(fl, flags.p, sizeof fl, st))) return fail(rc);
+    const bool rows_fit = fl[1] == 0 && fl[0] > 0 && nn_max <= 128 && (size_t)fl[0] * 72 * ROW_WAVES <= 64 * 1024;
+    if (kind >= 0) {
+        if ((kind == CSR_ROWS && !rows_fit) || (kind == CSR_SHORT && fl[0] > SHORT_ROW))
+            return fail(set_error(YETI_ERR_INVALID_ARGUMENT, "CSR: the values of this model cannot be gathered in way %d", kind));
+        c->kind = (CsrValues)kind;
+    } else if (long_rows && rows_fit) {
+        c->kind = CSR_ROWS;
+    } else if (mean <= SHORT_ROW && 4 * fl[3] < fl[2]) {
+        c->kind = CSR_EVERY;
+    } else if (mean <= SHORT_ROW && fl[0] <= SHORT_ROW) {
+        c->kind = CSR_SHORT;
+    }
+    if (c->kind == CSR_ROWS) {
+        c->upper = fl[0];
         c->sstride = nn_max;
-        if (flags.alloc(2) != hipSuccess || hipMemsetAsync(flags.p, 0, 8, st) != hipSuccess ||
-            c->irow.alloc(std::max<int64_t>(ninc, 1)) != hipSuccess ||
-            c->slots.alloc((size_t)std::max<int64_t>(ninc, 1) * nn_max) != hipSuccess)
+        if (c->irow.alloc(std::max<int64_t>(ninc, 1)) != hipSuccess ||
+            c->slots.alloc((size_t)std::max<int64_t>(ninc, 1) * nn_max) != hipSuccess ||
+            c->iptr.alloc(v.nb_cp + 1) != hipSuccess ||
+            hipMemcpyAsync(c->iptr.p, inc_ptr.p, 8 * (size_t)(v.nb_cp + 1), hipMemcpyDeviceToDevice, st) != hipSuccess)
             return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc element rows"));
         hipLaunchKernelGGL(slot_kernel, dim3(v.nb_cp), dim3(64), 0, st, v.nb_cp, inc_ptr.p, inc.p, pi, c->bptr.p, c->bcol.p,
-                           c->bdiag.p, c->sstride, c->irow.p, c->slots.p, flags.p);
-        if (hipMemcpyAsync(fl, flags.p, 8, hipMemcpyDeviceToHost, st) != hipSuccess ||
-            hipStreamSynchronize(st) != hipSuccess)
-            return fail(set_error(YETI_ERR_DEVICE, "CSR: copy failed"));
-        if (fl[1] == 0 && (size_t)fl[0] * 72 * ROW_WAVES <= 64 * 1024) {
-            c->upper = fl[0];
-            if (c->iptr.alloc(v.nb_cp + 1) != hipSuccess ||
-                hipMemcpyAsync(c->iptr.p, inc_ptr.p, 8 * (size_t)(v.nb_cp + 1), hipMemcpyDeviceToDevice, st) != hipSuccess)
-                return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc element rows"));
-        } else {
-            c->irow.release();
-            c->slots.release();
+                           c->bdiag.p, c->sstride, c->irow.p, c->slots.p);
+    } else {   // contributions per listed block
+        const bool dense = c->kind == CSR_LIST;
+        const int64_t *lptr = c->bptr.p;
+        c->nlist = c->nblocks;
+        if (dense) {
+            if (c->uptr.alloc(v.nb_cp + 1) != hipSuccess) return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc block list"));
+            if ((rc = exclusive_scan<int32_t>(rowlen.p, v.nb_cp, c->uptr.p, st))) return fail(rc);
+            if ((rc = read_back(&c->nlist, c->uptr.p + v.nb_cp, 8, st))) return fail(rc);
+            lptr = c->uptr.p;
         }
-    }
-    // contributions per block
-    if (c->upper == 0) {
-        if (bcount.alloc(std::max<int64_t>(c->nblocks, 1)) != hipSuccess ||
-            c->cptr.alloc(c->nblocks + 1) != hipSuccess)
+        const int64_t nl = std::max<int64_t>(c->nlist, 1);
+        if (bcount.alloc(nl) != hipSuccess || c->cptr.alloc(c->nlist + 1) != hipSuccess ||
+            (c->kind != CSR_SHORT && c->urow.alloc(nl) != hipSuccess))
             return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc contributions"));
-        hipLaunchKernelGGL(contrib_kernel<false>, dim3(v.nb_cp), dim3(64), 0, st, v.nb_cp, inc_ptr.p, inc.p, pi,
-                           c->bptr.p, c->bcol.p, bcount.p, nullptr, nullptr);
-        if ((rc = exclusive_scan<int32_t>(bcount.p, c->nblocks, c->cptr.p, st))) return fail(rc);
+        if (c->kind != CSR_SHORT)
+            hipLaunchKernelGGL(list_rows_kernel, dim3((v.nb_cp + 3) / 4), dim3(256), 0, st, v.nb_cp, lptr, c->urow.p);
+        const int32_t *first = c->kind == CSR_EVERY ? nullptr : c->bdiag.p;
+        hipLaunchKernelGGL(contrib_kernel<false>, dim3(v.nb_cp), dim3(64), 0, st, v.nb_cp, inc_ptr.p, inc.p, pi, c->bptr.p,
+                           c->bcol.p, first, lptr, dense, bcount.p, nullptr, nullptr);
+        if ((rc = exclusive_scan<int32_t>(bcount.p, c->nlist, c->cptr.p, st))) return fail(rc);
         int64_t ncontrib = 0;
-        if (hipMemcpy(&ncontrib, c->cptr.p + c->nblocks, 8, hipMemcpyDeviceToHost) != hipSuccess)
-            return fail(set_error(YETI_ERR_DEVICE, "CSR: copy failed"));
+        if ((rc = read_back(&ncontrib, c->cptr.p + c->nlist, 8, st))) return fail(rc);
         if (c->contrib.alloc(std::max<int64_t>(ncontrib, 1)) != hipSuccess)
             return fail(set_error(YETI_ERR_DEVICE, "CSR: alloc contrib list (%lld entries)", (long long)ncontrib));
-        hipLaunchKernelGGL(contrib_kernel<true>, dim3(v.nb_cp), dim3(64), 0, st, v.nb_cp, inc_ptr.p, inc.p, pi,
-                           c->bptr.p, c->bcol.p, nullptr, c->cptr.p, c->contrib.p);
+        hipLaunchKernelGGL(contrib_kernel<true>, dim3(v.nb_cp), dim3(64), 0, st, v.nb_cp, inc_ptr.p, inc.p, pi, c->bptr.p,
+                           c->bcol.p, first, lptr, dense, nullptr, c->cptr.p, c->contrib.p);
     }
     // scalar pattern
     if (c->rowptr.alloc(3 * (int64_t)v.nb_cp + 1) != hipSuccess ||
@@ -827,6 +922,10 @@ int32_t yeti_csr_create(const yeti_asm *h, void *stream, yeti_csr **out) {
     return 0;
 }
 
+int32_t yeti_csr_create(const yeti_asm *h, void *stream, yeti_csr **out) { return yeti_csr_create_as(h, -1, stream, out); }
+
+int32_t yeti_csr_values_kind(const yeti_csr *c) { return c ? (int32_t)c->kind : -1; }
+
 int64_t yeti_csr_nnz(const yeti_csr *c) { return c ? 9 * c->nblocks : -1; }
 int32_t yeti_csr_nrows(const yeti_csr *c) { return c ? 3 * c->nb_cp : -1; }
 const int64_t *yeti_csr_rowptr(const yeti_csr *c) { return c ? c->rowptr.p : nullptr; }
@@ -835,7 +934,7 @@ const int32_t *yeti_csr_colind(const yeti_csr *c) { return c ? c->colind.p : nul
 int32_t yeti_csr_values(const yeti_csr *c, const double *Kdata_dev, double *vals_dev, void *stream) {
     if (!c || !Kdata_dev || !vals_dev) return set_error(YETI_ERR_INVALID_ARGUMENT, "null argument");
     if (c->nblocks == 0) return 0;
-    if (c->upper > 0) {
+    if (c->kind == CSR_ROWS) {
         auto rows = [&](auto kern) {
             hipLaunchKernelGGL(kern, dim3(xcd_grid(((int64_t)c->nb_cp + ROW_WAVES - 1) / ROW_WAVES)), dim3(64 * ROW_WAVES),
                                (size_t)c->upper * 72 * ROW_WAVES, (hipStream_t)stream, c->nb_cp, c->upper, c->sstride,
@@ -847,17 +946,21 @@ int32_t yeti_csr_values(const yeti_csr *c, const double *Kdata_dev, double *vals
         YETI_HIP(hipGetLastError());
         return 0;
     }
-    // lanes per row: the mean number of its blocks J >= I (p = 1: 14 of a row's 27), so that short rows
-    // share a wave
-    const int64_t mean = (c->nblocks / std::max(c->nb_cp, 1) + 1) / 2;
-    auto go = [&](auto kern, int rows) {
-        hipLaunchKernelGGL(kern, dim3(xcd_grid(((int64_t)c->nb_cp + rows - 1) / rows)), dim3(256), 0, (hipStream_t)stream,
-                           c->nb_cp, c->bptr.p, c->bcol.p, c->bdiag.p, c->mirror.p, c->cptr.p, c->contrib.p, Kdata_dev,
-                           vals_dev);
+    const int64_t nitem = c->kind == CSR_SHORT ? (int64_t)SHORT_ROW * c->nb_cp : c->nlist;
+    auto go = [&](auto kern, int vt) {
+        hipLaunchKernelGGL(kern, dim3(xcd_grid((nitem + vt - 1) / vt)), dim3(vt), 160 * vt, (hipStream_t)stream, nitem,
+                           c->kind == CSR_LIST ? c->uptr.p : c->bptr.p, c->urow.p, c->bptr.p, c->bcol.p, c->bdiag.p,
+                           c->mirror.p, c->cptr.p, c->contrib.p, Kdata_dev, vals_dev);
     };
-    if (mean <= 16) go(csr_values_kernel<16>, 16);
-    else if (mean <= 32) go(csr_values_kernel<32>, 8);
-    else go(csr_values_kernel<64>, 4);
+    // Small workgroups spread short lists over the CUs (4^3 p = 3: 24.7 -> 20.1 us); long ones are 1 %
+    // faster in larger ones. The LDS is not used: 160 bytes per thread let 4 waves onto a SIMD, where 6
+    // evict more of what their neighbours read from L2 (90^3 p = 1 1343 -> 1261 us, 16^3 p = 4 1374 -> 1290).
+    const bool small = nitem <= 1 << 21;
+    switch (c->kind) {
+    case CSR_SHORT: small ? go(csr_values_kernel<64, CSR_SHORT>, 64) : go(csr_values_kernel<256, CSR_SHORT>, 256); break;
+    case CSR_EVERY: small ? go(csr_values_kernel<64, CSR_EVERY>, 64) : go(csr_values_kernel<256, CSR_EVERY>, 256); break;
+    default: small ? go(csr_values_kernel<64, CSR_LIST>, 64) : go(csr_values_kernel<256, CSR_LIST>, 256); break;
+    }
     YETI_HIP(hipGetLastError());
     return 0;
 }

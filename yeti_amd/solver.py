@@ -17,11 +17,16 @@ from .assembly import Assembler, _stream_handle
 
 
 class StiffnessCSR:
-    def __init__(self, asm: Assembler, stream=None):
+    """The CSR of one assembled model. ``kind``: how the values are gathered (0 element rows, 1 short
+    rows, 2 blocks J >= I, 3 every block); None takes what suits the model. All give the same bits."""
+
+    def __init__(self, asm: Assembler, stream=None, kind=None):
         self.asm = asm
         h = C.c_void_p()
-        _lib.check(_lib.lib().yeti_csr_create(asm._h, _stream_handle(stream), C.byref(h)))
+        _lib.check(_lib.lib().yeti_csr_create_as(asm._h, -1 if kind is None else int(kind), _stream_handle(stream),
+                                                 C.byref(h)))
         self._h = h
+        self.kind = int(_lib.lib().yeti_csr_values_kind(h))
         self.nnz = int(_lib.lib().yeti_csr_nnz(h))
         self.nrows = int(_lib.lib().yeti_csr_nrows(h))
         self.rowptr_ptr = _lib.lib().yeti_csr_rowptr(h)
