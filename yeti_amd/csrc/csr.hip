@@ -562,8 +562,8 @@ row_values_kernel(int32_t nb_cp, int32_t upper, int32_t sstride, const int64_t *
                 p[3 * kk + ll] += kk == ll ? 2.0 * v[u] : v[u];
                 if (kk != ll) p[3 * ll + kk] += v[u];
             }
-            wave_lds_sync();   // the next step's lanes may add to these addresses
         }
+        wave_lds_sync();   // other lanes may add the next run's entries to these addresses (a run's are distinct)
 #pragma unroll
         for (int u = 0; u < RG; ++u) v[u] = w[u];
 #pragma unroll
