@@ -729,10 +729,10 @@ struct PatchDev {
     int nelem;
     double lam, mu, rho;
     bool u1;
-    DevBuf<double> U[3];
-    // 1D basis tables per knot span, padded to tab_n = max degree + 1 functions (basis_table);
-    // tab_n = 0: no active element
-    DevBuf<double> tab[3];
+    // knot vectors, and 1D basis tables per knot span, padded to tab_n = max degree + 1 functions
+    // (basis_table; tab_n = 0: no active element), in one buffer
+    DevBuf<double> knots;
+    const double *U[3] = {nullptr, nullptr, nullptr}, *tab[3] = {nullptr, nullptr, nullptr};
     int tab_n = 0;
     DevBuf<int32_t> ien, nijk, elems;
     DevBuf<double> weight;
@@ -834,10 +834,9 @@ static bool kernel_available(int p0, int p1, int p2, int ng) {
 // padded with zeros to N, and their derivatives at ng Gauss points, [B | dB][g][i] in reversed local
 // index (shap.f90:94-119), and half the span's length; 2 ng N + 2 values per span.
 template <int P>
-static void basis_table_p(const double *U, int nkv, int N, int ng, std::vector<double> &tab) {
+static void basis_table_p(const double *U, int nkv, int N, int ng, const double *gx, std::vector<double> &tab) {
     const int rec = 2 * ng * N + 2;
-    double gx[MAX_NG], gw[MAX_NG], B[P + 1], dB[P + 1];
-    gauss_legendre(ng, gx, gw);
+    double B[P + 1], dB[P + 1];
     tab.assign((size_t)rec * std::max(nkv - 1, 1), 0.0);
     for (int i = P; i + P + 1 < nkv; ++i) {
         const double u0 = U[i], u1 = U[i + 1];
@@ -854,12 +853,12 @@ static void basis_table_p(const double *U, int nkv, int N, int ng, std::vector<d
     }
 }
 
-static void basis_table(int p, const double *U, int nkv, int N, int ng, std::vector<double> &tab) {
+static void basis_table(int p, const double *U, int nkv, int N, int ng, const double *gx, std::vector<double> &tab) {
     switch (p) {
-    case 1: basis_table_p<1>(U, nkv, N, ng, tab); break;
-    case 2: basis_table_p<2>(U, nkv, N, ng, tab); break;
-    case 3: basis_table_p<3>(U, nkv, N, ng, tab); break;
-    default: basis_table_p<4>(U, nkv, N, ng, tab); break;
+    case 1: basis_table_p<1>(U, nkv, N, ng, gx, tab); break;
+    case 2: basis_table_p<2>(U, nkv, N, ng, gx, tab); break;
+    case 3: basis_table_p<3>(U, nkv, N, ng, gx, tab); break;
+    default: basis_table_p<4>(U, nkv, N, ng, gx, tab); break;
     }
 }
 
@@ -899,7 +898,7 @@ static GenArgs general_args(yeti_asm *h, PatchDev &pd) {
     ga.weight = pd.weight.p;
     ga.nijk = pd.nijk.p;
     for (int d = 0; d < 3; ++d) {
-        ga.tab[d] = pd.tab[d].p;
+        ga.tab[d] = pd.tab[d];
         ga.n[d] = pd.p[d] + 1;
     }
     ga.elems = pd.elems.p;
@@ -927,9 +926,9 @@ static int launch_elem(yeti_asm *h, PatchDev &pd, const double *coords, double *
     pa.ien = pd.ien.p;
     pa.weight = pd.weight.p;
     pa.nijk = pd.nijk.p;
-    pa.U0 = pd.U[0].p;
-    pa.U1 = pd.U[1].p;
-    pa.U2 = pd.U[2].p;
+    pa.U0 = pd.U[0];
+    pa.U1 = pd.U[1];
+    pa.U2 = pd.U[2];
     pa.lam = pd.lam;
     pa.mu = pd.mu;
     gauss_legendre(NG, pa.g.x, pa.g.w);
@@ -1240,9 +1239,9 @@ static int launch_mass(yeti_asm *h, PatchDev &pd, double *Md, int32_t *Mr, int32
     pa.ien = pd.ien.p;
     pa.weight = pd.weight.p;
     pa.nijk = pd.nijk.p;
-    pa.U0 = pd.U[0].p;
-    pa.U1 = pd.U[1].p;
-    pa.U2 = pd.U[2].p;
+    pa.U0 = pd.U[0];
+    pa.U1 = pd.U[1];
+    pa.U2 = pd.U[2];
     pa.elems = pd.elems.p;
     pa.offs = pd.offs.p;
     pa.n_active = pd.n_active;
@@ -1661,7 +1660,7 @@ static void launch_grad(yeti_asm *h, PatchDev &pd, const GradFields &gf, int64_t
     ga.weight = pd.weight.p;
     ga.nijk = pd.nijk.p;
     for (int d = 0; d < 3; ++d) {
-        ga.tab[d] = pd.tab[d].p;
+        ga.tab[d] = pd.tab[d];
         ga.n[d] = pd.p[d] + 1;
     }
     ga.elems = pd.elems.p;
@@ -1693,9 +1692,9 @@ static int launch_grad_kind(yeti_asm *h, PatchDev &pd, const GradFields &gf, int
         pa.ien = pd.ien.p;
         pa.weight = pd.weight.p;
         pa.nijk = pd.nijk.p;
-        pa.U0 = pd.U[0].p;
-        pa.U1 = pd.U[1].p;
-        pa.U2 = pd.U[2].p;
+        pa.U0 = pd.U[0];
+        pa.U1 = pd.U[1];
+        pa.U2 = pd.U[2];
         pa.elems = pd.elems.p;
         pa.n_active = pd.n_active;
         pa.lam = pd.lam;
@@ -1842,7 +1841,7 @@ static int run_load_grad(yeti_asm *h, const double *u, double *g, hipStream_t st
         rp.weight = pd->weight.p;
         rp.nijk = pd->nijk.p;
         for (int d = 0; d < 3; ++d) {
-            rp.U[d] = pd->U[d].p;
+            rp.U[d] = pd->U[d];
             rp.p[d] = pd->p[d];
         }
         rp.elems = pd->loaded.p;
@@ -1936,7 +1935,7 @@ static int run_rhs(yeti_asm *h, double *F, hipStream_t st) {
         rp.weight = pd->weight.p;
         rp.nijk = pd->nijk.p;
         for (int d = 0; d < 3; ++d) {
-            rp.U[d] = pd->U[d].p;
+            rp.U[d] = pd->U[d];
             rp.p[d] = pd->p[d];
         }
         rp.ng = pd->ng;
@@ -2063,14 +2062,26 @@ static int create(const yeti_system_inputs *in, int layout, yeti_asm **out) {
         pd->n_active = (int32_t)act.size();
         hipError_t e1 = hipSuccess;
         pd->tab_n = act.empty() ? 0 : std::max(std::max(pd->p[0], pd->p[1]), pd->p[2]) + 1;
-        for (int d = 0; d < 3 && e1 == hipSuccess; ++d) {
-            e1 = pd->U[d].upload(in->Ukv + kv, nkv[d]);
-            if (e1 == hipSuccess && pd->tab_n > 0) {
-                std::vector<double> tab;
-                basis_table(pd->p[d], in->Ukv + kv, nkv[d], pd->tab_n, pd->ng, tab);
-                e1 = pd->tab[d].upload(tab.data(), tab.size());
+        {
+            std::vector<double> k, tab;
+            size_t at[6] = {0, 0, 0, 0, 0, 0};
+            for (int d = 0; d < 3; ++d) {
+                at[d] = k.size();
+                k.insert(k.end(), in->Ukv + kv, in->Ukv + kv + nkv[d]);
+                kv += nkv[d];
             }
-            kv += nkv[d];
+            double gx[MAX_NG], gw[MAX_NG];
+            if (pd->tab_n > 0) gauss_legendre(pd->ng, gx, gw);
+            for (int d = 0; d < 3 && pd->tab_n > 0; ++d) {
+                basis_table(pd->p[d], k.data() + at[d], nkv[d], pd->tab_n, pd->ng, gx, tab);
+                at[3 + d] = k.size();
+                k.insert(k.end(), tab.begin(), tab.end());
+            }
+            e1 = pd->knots.upload(k.data(), k.size());
+            for (int d = 0; d < 3; ++d) {
+                pd->U[d] = pd->knots.p + at[d];
+                if (pd->tab_n > 0) pd->tab[d] = pd->knots.p + at[3 + d];
+            }
         }
         if (e1 == hipSuccess) e1 = pd->ien.upload(in->IEN + ieoff, (size_t)pd->nnode * pd->nelem);
         if (e1 == hipSuccess) e1 = pd->weight.upload(in->weight + woff, (size_t)nn_geo * pd->nelem);
