@@ -1,10 +1,10 @@
-"""The general-degree element path (elem_generic_kernel): degree triples and Gauss orders the
-MFMA element kernel is not built for -- unequal degrees per direction, NBINT other than
-(p + 1)^3 -- against the oracle (COO indices bit-exact, values and F within 1e-12 of their
-maximum), in the serial (packed) and OpenMP (slotted) layouts of the drop-ins, and the
-consistent mass matrix, the natural-frequency gradient (run-time-degree instance of the
-gradient kernel), the VTU vertex fields and the displacement at parametric points on the same
-cases.
+"""The general element kernel (elem_general.hip; p = 3 with 4 points has a stiffness kernel of its own,
+p = 3 and 4 with p + 1 points a mass kernel) on degree triples and Gauss orders that only it takes -- unequal
+degrees per direction, NBINT other than (p + 1)^3 -- against the oracle (COO indices bit-exact,
+values and F within 1e-12 of their maximum), in the serial (packed) and OpenMP (slotted) layouts of
+the drop-ins, and the consistent mass matrix, the shape gradients (factorised at max(p) + 1 points,
+the run-time-order kernel at others), the VTU vertex fields and the displacement at parametric
+points on the same cases.
 """
 import os
 
@@ -39,7 +39,7 @@ CASES = {
 
 
 def test_cases_take_the_general_path():
-    """Every case here is one the MFMA kernel is not built for (equal degrees, p + 1 points)."""
+    """No case here has the equal degrees and p + 1 points that other kernels are built for."""
     for name, make in CASES.items():
         a = make()
         from yeti_amd._abi import args_to_dict
@@ -154,6 +154,39 @@ def test_gpu_general_degrees_strain_energy_grad(name):
         fd = -(_energy(dp, u) - _energy(dm, u)) / (2 * h)
         an = float(g @ dX.T.reshape(-1))
         assert abs(fd - an) <= 1e-6 * np.linalg.norm(g) * np.linalg.norm(dX), (fd, an)
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("name,make", [("p=3, 4 points", lambda: box(3, 4)), ("p=4, 5 points", lambda: box(4, 5)),
+                                       ("degrees (2,3,1)", CASES["beam degrees (2,3,1)"]),
+                                       ("p=3, 3 points", lambda: box(3, 3)), ("p=1, 3 points", lambda: box(1, 3))])
+def test_gpu_work_gradients_of_different_fields(name, make):
+    """grad_lin_elast_work for a state and 5 adjoints that differ from it (more than one launch
+    takes), factorised and with run-time orders: -a^T (dK/dX) u by polarisation,
+    (E(u - a) - E(u + a)) / 4 with E(v) = v^T (dK/dX) v from the oracle's natural-frequency gradient
+    at eigenvalue 0 times v^T M v, within 1e-11 of the maximum."""
+    import torch
+    from yeti_amd._abi import args_to_dict
+    from yeti_amd.assembly import Assembler
+    print("[case] work gradients of different fields: %s" % name, flush=True)
+    d = args_to_dict(make())
+    d["RHO"] = np.full(int(np.asarray(d["nb_elem_patch"]).size), 7.8)
+    ncp = int(np.asarray(d["COORDS3D"]).shape[1])
+    rng = np.random.default_rng(8)
+    u, adj = rng.standard_normal(3 * ncp), rng.standard_normal((5, 3 * ncp))
+    asm = Assembler(d)
+    try:
+        g = asm.grad_lin_elast_work(torch.from_numpy(u).cuda(), torch.from_numpy(adj).cuda())[0].cpu().numpy()
+    finally:
+        asm.close()
+    v = np.concatenate([u - adj, u + adj])
+    M, rm, cm = O.oracle_mass_coo(d)
+    mass = 2.0 * (v[:, rm] * v[:, cm]) @ M
+    E = O.oracle_grad_vibration(d, v.reshape(10, ncp, 3).transpose(0, 2, 1), np.zeros(10))
+    E = E.transpose(0, 2, 1).reshape(10, 3 * ncp) * mass[:, None]
+    go = (E[:5] - E[5:]) / 4
+    for k in range(5):
+        assert np.abs(g[k] - go[k]).max() <= 1e-11 * np.abs(go[k]).max(), k
 
 
 @pytest.mark.gpu

@@ -476,7 +476,7 @@ def test_work_gradients_on_another_stream_keep_their_inputs(gpu):
 
 def test_32cube_p2_gradient(gpu):
     """The differentiation workload at its size: 32^3 elements, p = 2 (39,304 control points).
-    * gradlinelastwork_an (element-wise gradient kernel, polarised) and the matrix-free MODE 2
+    * gradlinelastwork_an (element-wise gradient kernel) and the matrix-free MODE 2
       strain-energy gradient against the compiled gradLinElastWork_AN (tests/golden/
       grad_32cube_p2.npz: 8,192 sampled control points x 3 directions x 2 adjoints, and the full
       arrays' Frobenius norms): within 1e-10 of the maximum;
