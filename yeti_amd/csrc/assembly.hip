@@ -1027,10 +1027,10 @@ struct MassCfg {
     static constexpr int NP1 = P + 1, NN = NP1 * NP1 * NP1, NQ = NG * NG * NG;
     static constexpr int NNP = (NN + 15) / 16 * 16, NT = NNP / 16, NTILE = NT * (NT + 1) / 2;
     static constexpr int MAXT = (NTILE + 3) / 4;                       // tiles per wave
-    // points per chunk: at most 32, so that at p = 3 the LDS (26 KB) and registers (compiled for
+    // points per chunk: 32, so that at p = 3 the LDS (26 KB) and registers (compiled for
     // 4 waves per SIMD) allow 4 workgroups per CU (64-point chunks: 49 KB, 3 per CU, 16.6 ms
     // against 15.5 ms at 64^3)
-    static constexpr int MQC = NQ <= 32 ? (NQ + 7) / 8 * 8 : 32;
+    static constexpr int MQC = 32;
     static constexpr int G = 256 / MQC;                                // threads per point
     static constexpr int RS = MQC + 2;                                 // R row stride (doubles)
     static constexpr int NPAIR = NN * (NN + 1) / 2;
@@ -1040,7 +1040,6 @@ struct MassCfg {
     static constexpr int N_U = NNP * RS + 2 * MQC * 3 * NP1;
     static constexpr int NDBL = O_U + (N_U > NPAIR ? N_U : NPAIR);
     static constexpr int64_t NCOO = coo_start(NN);
-    static_assert(256 % MQC == 0 && MQC % 8 == 0 && G <= 64, "mass chunking");
 };
 
 template <int P, int NG, bool WRITE_IDX>

@@ -13,12 +13,13 @@ struct ElemCfg {
     static constexpr int NP1 = P + 1;
     static constexpr int NN = NP1 * NP1 * NP1;          // nodes (CPs) per element
     static constexpr int NQ = NG * NG * NG;             // Gauss points per element
-    // the record of an element: 12 geometry values per Gauss point ([v][q]), the 1D basis tables B,
-    // dB ([which][d][g][i]), the node weights and the nodes' dof bases 3 (IEN - 1) (int32, from double
-    // offset DOFOFF)
+    // the record of an element: 12 geometry values per Gauss point ([v][q]); at p = 3 then the 1D basis
+    // tables B, dB ([which][d][g][i]), the node weights and the nodes' dof bases 3 (IEN - 1) (int32,
+    // from double offset DOFOFF), which elem_general_kernel fetches itself
+    static constexpr bool NODES = P == 3;
     static constexpr int NTAB = 2 * 3 * NG * NP1;
     static constexpr int64_t DOFOFF = (int64_t)ELEM_NGEO * NQ + NTAB + NN;
-    static constexpr int64_t REC = DOFOFF + (NN + 1) / 2;
+    static constexpr int64_t REC = NODES ? DOFOFF + (NN + 1) / 2 : (int64_t)ELEM_NGEO * NQ;
 };
 
 __host__ __device__ constexpr int64_t coo_start(int b) { return (9LL * b * b + 3LL * b) / 2; }
@@ -39,9 +40,10 @@ struct PatchArgs {
 // ---------------------------------------------------------------------------------------
 // Geometry pass: per active element gi a record of REC doubles at geo + gi REC: for Gauss point
 // q, [v NQ + q] with v = 3 m + c: A[m][c] = sqrt(w |det J|) / W dxi_m/dx_c; v = 9 + m:
-// dW/dxi_m / W; then the element's 1D basis tables (values and derivatives at the abscissae,
-// reversed local index), its node weights and its nodes' dof bases. J is the derivative with respect to the knot parameters (shap.f90:133-153); w |det J| includes the
-// parent-to-parameter factors (shap.f90:156-178) and the Gauss weights (UELMAT.f90:118-119).
+// dW/dxi_m / W; at p = 3 then the element's 1D basis tables (values and derivatives at the abscissae,
+// reversed local index), its node weights and its nodes' dof bases. J is the derivative with respect
+// to the knot parameters (shap.f90:133-153); w |det J| includes the parent-to-parameter factors
+// (shap.f90:156-178) and the Gauss weights (UELMAT.f90:118-119).
 // One wave per element, 4 per workgroup. The 16 sums a Gauss point needs (W, dW/dxi_m, and
 // sum w x_c R and its xi derivatives, before the division by W) are tensor-product contractions
 // of the four nodal quantities (w, w x, w y, w z), evaluated by sum factorisation through LDS:
@@ -69,12 +71,14 @@ __global__ void __launch_bounds__(256) elem_geo_kernel(PatchArgs pa, double *__r
             const int32_t cp1 = pa.ien[(int64_t)NN * e + a];
             const double *xp = pa.coords + 3 * (int64_t)(cp1 - 1);
             const double w = pa.weight[(int64_t)NN * e + a];
-            reinterpret_cast<int32_t *>(rec + C::DOFOFF)[a] = 3 * (cp1 - 1);
+            if (C::NODES) {
+                reinterpret_cast<int32_t *>(rec + C::DOFOFF)[a] = 3 * (cp1 - 1);
+                rec[ELEM_NGEO * NQ + C::NTAB + a] = w;
+            }
             cp[wv][0][a] = w;
             cp[wv][1][a] = w * xp[0];
             cp[wv][2][a] = w * xp[1];
             cp[wv][3][a] = w * xp[2];
-            rec[ELEM_NGEO * NQ + C::NTAB + a] = w;
         }
         if (lane < 3 * NG) {   // 1D bases of direction d at abscissa g
             const int d = lane / NG, g = lane - d * NG;
@@ -84,13 +88,15 @@ __global__ void __launch_bounds__(256) elem_geo_kernel(PatchArgs pa, double *__r
             const double u = ((u1 - u0) * pa.g.x[g] + (u1 + u0)) * 0.5;
             double N[NP1], dN[NP1];
             bspline_ders<P>(span1 - 1, u, U, N, dN);
-            double *tb = rec + ELEM_NGEO * NQ + (d * NG + g) * NP1;
 #pragma unroll
             for (int i = 0; i < NP1; ++i) {   // local index i <-> basis function P - i
                 tab[wv][d][0][g][i] = N[P - i];
                 tab[wv][d][1][g][i] = dN[P - i];
-                tb[i] = N[P - i];
-                tb[3 * NG * NP1 + i] = dN[P - i];
+                if (C::NODES) {
+                    double *tb = rec + ELEM_NGEO * NQ + (d * NG + g) * NP1;
+                    tb[i] = N[P - i];
+                    tb[3 * NG * NP1 + i] = dN[P - i];
+                }
             }
             if (g == 0) hh[wv][d] = 0.5 * (u1 - u0);
         }
