@@ -20,6 +20,7 @@
 #include <vector>
 
 #include "common.hpp"
+#include "coo_entries.hpp"
 #include "elem_general.hpp"
 #include "elem_p3.hpp"
 
@@ -1039,7 +1040,7 @@ struct MassCfg {
     static constexpr int O_B = O_U + NNP * RS, O_DB = O_B + MQC * 3 * NP1;
     static constexpr int N_U = NNP * RS + 2 * MQC * 3 * NP1;
     static constexpr int NDBL = O_U + (N_U > NPAIR ? N_U : NPAIR);
-    static constexpr int64_t NCOO = coo_start(NN);
+    static constexpr int NCOO = coo_start(NN);
 };
 
 template <int P, int NG, bool WRITE_IDX>
@@ -1203,9 +1204,9 @@ mass_kernel(PatchArgs pa, double rho, double *__restrict__ Md,
         // emission: entry x of the element's range lies in column b with start(b) <= x < start(b+1)
         const int64_t base = pa.offs[gi];
         int b = 0;
-        for (int x = t; x < (int)C::NCOO; x += 256) {
-            while (b + 1 < NN && (int)coo_start(b + 1) <= x) ++b;
-            const unsigned r = (unsigned)(x - (int)coo_start(b));
+        for (int x = t; x < C::NCOO; x += 256) {
+            while (b + 1 < NN && coo_start(b + 1) <= x) ++b;
+            const unsigned r = (unsigned)(x - coo_start(b));
             const int mb = b * (b + 1) / 2;
             double v;
             int32_t row, col;

@@ -8,6 +8,7 @@
 // order of build_system_elemStorage.f90:260-293.
 #include <algorithm>
 
+#include "coo_entries.hpp"
 #include "copy_out.hpp"
 #include "elem_general.hpp"
 
@@ -76,30 +77,17 @@ __device__ __forceinline__ double parts_sum(double v) {
 // x / n for x < 1024, n <= 81 with m = ceil(65536 / n): x (m n - 65536) < 65536
 __device__ __forceinline__ int div_by(int x, int m) { return (x * m) >> 16; }
 
-__host__ __device__ constexpr int gen_coo_start(int b) { return (9 * b * b + 3 * b) / 2; }
-
-// dofs of COO entry x of an element (any node count): 3 a + kk | (3 b + ll) << 8
-struct EntryTab {
-    alignas(16) uint16_t v[gen_coo_start(GEN_MAXN)];
-    constexpr EntryTab() : v() {
-        int x = 0;
-        for (int b = 0; b < GEN_MAXN; ++b)
-            for (int a = 0; a <= b; ++a)
-                for (int l = 0; l < 3; ++l)
-                    for (int k = 0; k < (a < b ? 3 : l + 1); ++k) v[x++] = (uint16_t)((3 * a + k) | (3 * b + l) << 8);
-    }
-};
-__device__ constexpr EntryTab entry_tab{};
-static_assert(gen_coo_start(16) % 8 == 0 && gen_coo_start(32) % 8 == 0 && gen_coo_start(48) % 8 == 0 &&
-                  gen_coo_start(GEN_MAXN) % 8 == 0,
+static_assert(GEN_MAXN == ENTRY_NODES, "entry_tab holds every element");
+static_assert(coo_start(16) % 8 == 0 && coo_start(32) % 8 == 0 && coo_start(48) % 8 == 0 &&
+                  coo_start(GEN_MAXN) % 8 == 0,
               "the rounds' table rows are copied 16 bytes at a time");
 
 // Largest number of entries of a round: the whole element up to NT = 2, else a tile column
 template <int NT>
 __host__ __device__ constexpr int gen_round_entries(int nn) {
-    if (NT <= 2) return gen_coo_start(nn);
-    const int last = gen_coo_start(nn) - gen_coo_start(16 * (NT - 1));
-    const int prev = gen_coo_start(16 * (NT - 1)) - gen_coo_start(16 * (NT - 2));
+    if (NT <= 2) return coo_start(nn);
+    const int last = coo_start(nn) - coo_start(16 * (NT - 1));
+    const int prev = coo_start(16 * (NT - 1)) - coo_start(16 * (NT - 2));
     return last > prev ? last : prev;
 }
 
@@ -159,7 +147,7 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
             for (int x = t; x < (x1 - x0 + 7) / 8; x += NTH) reinterpret_cast<u32x4 *>(et)[x] = src[x];
         };
         constexpr int ROUNDS = NT <= 2 ? 1 : NT;
-        if (ROUNDS == 1 && MODE == 1) load_tab(0, gen_coo_start(NN));
+        if (ROUNDS == 1 && MODE == 1) load_tab(0, coo_start(NN));
         f64x4 acc[TILES];
 #pragma unroll
         for (int s = 0; s < TILES; ++s) acc[s] = f64x4{0.0, 0.0, 0.0, 0.0};
@@ -348,13 +336,13 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
         }
 #pragma unroll 1
         for (int rd = NT == 8 ? J0 : 0; rd < (NT == 8 ? J1 : ROUNDS); ++rd) {
-            const int x0 = ROUNDS == 1 ? 0 : gen_coo_start(16 * rd);
-            const int x1 = ROUNDS == 1 ? gen_coo_start(NN) : gen_coo_start(min(16 * rd + 16, NN));
+            const int x0 = ROUNDS == 1 ? 0 : coo_start(16 * rd);
+            const int x1 = ROUNDS == 1 ? coo_start(NN) : coo_start(min(16 * rd + 16, NN));
             if (ROUNDS > 1 && MODE == 1) load_tab(x0, x1);
             if (MODE == 0 && (ROUNDS == 1 || J == rd)) {
                 // register r of lane l holds row (l >> 4) + 4 r and column l & 15 of a tile
                 const int b = 16 * J + nl;
-                double *col = sm + gen_coo_start(b) - x0;
+                double *col = sm + coo_start(b) - x0;
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
                     const int a = 16 * I + 4 * r + kg;
@@ -408,7 +396,7 @@ elem_general_kernel(GenArgs ga, double *__restrict__ Kd, int32_t *__restrict__ K
                 if (IDX && NT == 8) {
                     // 9-bit dofs, which entry_tab does not hold: row by row
                     for (int b = 16 * rd + wv; b < min(16 * rd + 16, NN); b += C::WAVES) {
-                        int32_t *Rb = Re + gen_coo_start(b), *Cb = Ce + gen_coo_start(b);
+                        int32_t *Rb = Re + coo_start(b), *Cb = Ce + coo_start(b);
                         for (int y = lane; y < 9 * b + 6; y += 64) {
                             const int a = y < 9 * b ? y / 9 : b, m = y - 9 * a;
                             const int kk = a < b ? m % 3 : (0x210100 >> (4 * m)) & 15;

@@ -22,8 +22,6 @@ struct ElemCfg {
     static constexpr int64_t REC = NODES ? DOFOFF + (NN + 1) / 2 : (int64_t)ELEM_NGEO * NQ;
 };
 
-__host__ __device__ constexpr int64_t coo_start(int b) { return (9LL * b * b + 3LL * b) / 2; }
-
 struct PatchArgs {
     const double *coords;     // (3, nb_cp)
     const int32_t *ien;       // (nnode, nelem_patch), 1-based

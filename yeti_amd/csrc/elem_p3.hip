@@ -32,6 +32,7 @@
 #include <algorithm>
 #include <type_traits>
 
+#include "coo_entries.hpp"
 #include "copy_out.hpp"
 #include "elem_p3.hpp"
 
@@ -49,21 +50,7 @@ constexpr int CWAVES = 6, SWAVES = 2, NTH = 64 * (CWAVES + SWAVES);
 constexpr int SL = 64 * SWAVES;                        // store lanes
 constexpr int WORDS = NDE / 4, WPL = (WORDS + SL - 1) / SL;   // four entries each; per lane
 
-__host__ __device__ constexpr int start(int b) { return (9 * b * b + 3 * b) / 2; }
-static_assert(start(64) == NDE && start(48) == SPLIT, "COO layout");
-
-// dofs of entry x: 3 a + kk | (3 b + ll) << 8
-struct Tab {
-    alignas(16) uint16_t v[NDE];
-    constexpr Tab() : v() {
-        int x = 0;
-        for (int b = 0; b < 64; ++b)
-            for (int a = 0; a <= b; ++a)
-                for (int l = 0; l < 3; ++l)
-                    for (int k = 0; k < (a < b ? 3 : l + 1); ++k) v[x++] = (uint16_t)((3 * a + k) | (3 * b + l) << 8);
-    }
-};
-__device__ constexpr Tab tab{};
+static_assert(coo_start(64) == NDE && coo_start(48) == SPLIT, "COO layout");
 
 __device__ __forceinline__ f64x4 mm(double a, double b, f64x4 c) { return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0); }
 
@@ -130,7 +117,7 @@ elem_p3_kernel(const double *__restrict__ geo, const int64_t *__restrict__ offs,
     __shared__ __attribute__((aligned(16))) double wls[CWAVES][64];   // node weights, a copy per compute wave
     const int lane = threadIdx.x & 63, wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
     __shared__ __attribute__((aligned(16))) int32_t start8[64];   // byte offset of a node's row of entries
-    if (threadIdx.x < 64) start8[threadIdx.x] = 8 * start(threadIdx.x);
+    if (threadIdx.x < 64) start8[threadIdx.x] = 8 * coo_start(threadIdx.x);
     __syncthreads();
     const int64_t nidx = (int64_t)xcd_per(n) * XCDS;
     // element of step index s of this workgroup, -1 past the end of its XCD's run
@@ -307,7 +294,7 @@ elem_p3_kernel(const double *__restrict__ geo, const int64_t *__restrict__ offs,
         u32x2 rc[IDX ? WPL : 1];   // the dofs of four entries
         if (IDX) {
 #pragma unroll
-            for (int i = 0; i < WPL; ++i) rc[i] = *reinterpret_cast<const u32x2 *>(tab.v + 4 * min(cl + SL * i, WORDS - 1));
+            for (int i = 0; i < WPL; ++i) rc[i] = *reinterpret_cast<const u32x2 *>(entry_tab.v + 4 * min(cl + SL * i, WORDS - 1));
         }
         int32_t *dof = dofs[sw];
         // entries [x0, x1) of the element at base
