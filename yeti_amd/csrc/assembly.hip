@@ -1539,7 +1539,8 @@ __global__ void __launch_bounds__(256) shape_grad_rt_kernel(PatchArgs pa, GradFi
                             for (int k = 0; k < 3; ++k) {
                                 double v = m == k ? Wp : 0.0;
 #pragma unroll
-                                for (int i = 0; i < 3; ++i) v -= D[i][m] * sh[i][k] + H[i][m] * sd[i][k];
+                                for (int i = 0; i < 3; ++i)
+                                    v -= KIND == GRAD_MODES ? 2.0 * (D[i][m] * sd[i][k]) : D[i][m] * sh[i][k] + H[i][m] * sd[i][k];
                                 T[3 * m + k] = dv * v;
                             }
                         macc += uu * dv;
