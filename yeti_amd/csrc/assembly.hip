@@ -168,7 +168,7 @@ template <int MAXN>
 __device__ void rhs_basis(const RhsPatch &rp, int e, const double *pt, int nn, const double *sW,
                           const double (*sX)[3], double *R, double (*dR)[3], double AJ[3][3], double *detJ) {
     // R[c] (and, if dR is given, dR[c][m] = dR/d(parent coordinate m)) for the nodes a = lane + 64 c
-    // parametric point and 1D bases (degrees up to 8)
+    // parametric point and 1D bases (loaded elements' degrees, up to 4)
     const int lane = threadIdx.x;
     __shared__ double sb[3][10], sdb[3][10], shalf[3];
     if (lane < 3) {
@@ -303,9 +303,9 @@ static __device__ inline void rhs_basis_1d(int p, int i, double u, const double 
 //      and add them by shuffles; the first lane turns them into the point's load f_q / W;
 //   2. every thread owns a node (groups of threads split the chunk's points) and adds
 //      N_a(q) w_a f_q in registers.
-// 16x4x4 p=2 (16 elements, 9 points each) 7.0 us, 64^3 p=3 (4096 elements) 46 us
-// against one wave per element that walked the points one after the other with its node sums in
-// scratch memory.
+// 16x4x4 p=2 (16 elements, 9 points each) 41.8 -> 6.8 us, 64^3 p=3 (4096 elements) 233 -> 46 us, body
+// loads on all of 24^3 p=3 3752 -> 230 us, against one wave per element that walked the points one
+// after the other with its node sums in scratch memory.
 __global__ void __launch_bounds__(256) elem_rhs_kernel(RhsPatch rp, LoadTable lt, double *rhs_buf) {
     const int le = blockIdx.x;
     if (le >= rp.n_loaded) return;

@@ -26,9 +26,9 @@ typedef double f64x2 __attribute__((ext_vector_type(2)));
 // column J at a time) and copied by all threads front to back; their rows and columns come from
 // entry_tab. The mass keeps only M_ab, a <= b, in LDS and expands it on the way out.
 // Bound by FP64 issue (matrix and vector instructions do not overlap): 64^3 p = 2 takes 3.8 ms of its
-// 5.07 ms without the stores, whose floor is 2.1 ms; the mass at 61x53x47 p = 2 takes 1.0 of 2.12 ms.
+// 5.07 ms without the stores, whose floor is 2.1 ms; the mass at 61x53x47 p = 2 takes 1.0 of 1.99 ms.
 // Against vector sums of every node pair from LDS and block-wise stores: 45x14x11 degrees (2,3,1)
-// 1018 -> 216 us; mass 61x53x47 p = 2 2.94 -> 2.12 ms, 64^3 p = 1 1.91 -> 0.69 ms.
+// 1018 -> 216 us; mass 61x53x47 p = 2 2.61 -> 1.99 ms, 64^3 p = 1 1.91 -> 0.69 ms.
 // NT = 8 (125 nodes): 36 pairs of nine tiles are more accumulators than a CU has registers for, hence
 // four workgroups per element. Each builds G again and no two fit a CU (stage of 120 KB); at 23x18x13
 // the matrix instructions of the busiest SIMD take 1.6 of 3.76 ms (at 2.4 GHz). Against one persistent
